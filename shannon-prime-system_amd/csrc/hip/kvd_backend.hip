@@ -174,7 +174,7 @@ struct Uploader {                         // one allocation, arrays carved at 25
 
 int load_weight(const qwen3_model *qm, const gguf_tensor *t, int rows, int cols, Uploader &up,
                 std::vector<std::vector<int8_t>> &ebase_store, std::vector<std::vector<uint16_t>> &bs8_store,
-                DevW &w, size_t offs[4], int il) {
+                std::vector<std::vector<uint32_t>> &ex_store, DevW &w, size_t offs[7], int il) {
     if (!t) return fail("sp_hipkv_open: model lacks a weight tensor%s", "");
     const sp_arena_tensor *at = sp_arena_find(qm->arena, t->name);
     if (!at) return fail("sp_hipkv_open: weight %s not in the packed arena", t->name);
@@ -191,10 +191,11 @@ int load_weight(const qwen3_model *qm, const gguf_tensor *t, int rows, int cols,
     // the int64 accumulator (see kvd_gemv.hip) switch the tensor to int128
     // (8 zero bytes of padding: the GEMV reads a task's 8 rows in one load)
     ebase_store.emplace_back(rows + 8);
-    std::vector<int8_t> &eb = ebase_store.back();
+    ebase_store.emplace_back(rows);                        // largest block exponents (the folded GEMM)
+    std::vector<int8_t> &eb = ebase_store[ebase_store.size() - 2], &et = ebase_store.back();
     int lg = 0; while ((1 << lg) < (int)nb) lg++;
     const int max_spread = 21 - lg;
-    int wide = 0;
+    int wide = 0, fold = 1;
     for (int r = 0; r < rows; r++) {
         int emin = 127, emax = -127;
         const uint16_t *bs = p.bscale + (size_t)r * nb;
@@ -202,12 +203,32 @@ int load_weight(const qwen3_model *qm, const gguf_tensor *t, int rows, int cols,
             const int E5 = (bs[b] >> 10) & 31, mant = bs[b] & 1023;
             if (E5 == 31) return fail("sp_hipkv_open: %s has a non-finite block scale", t->name);
             if (!E5 && !mant) continue;
+            if (bs[b] & 0x8000) fold = 0;                  // its digits hold non-negative scales
             const int e = E5 ? E5 - 25 : -24;
             emin = std::min(emin, e); emax = std::max(emax, e);
         }
         if (emin > emax) emin = emax = 0;
         eb[r] = (int8_t)emin;
+        et[r] = (int8_t)emax;
+        if (emax - emin > 9) fold = 0;
         if (emax - emin > max_spread) wide = 1;
+    }
+    // blocks whose scale f16 2^(9 - emax) has a low byte, by 16-row tile
+    ex_store.emplace_back((size_t)(rows + 15) / 16 + 1, 0u);
+    ex_store.emplace_back();
+    if (fold) {
+        std::vector<uint32_t> &exo = ex_store[ex_store.size() - 2], &exl = ex_store.back();
+        for (int r = 0; r < rows; r++) {
+            const uint16_t *bs = p.bscale + (size_t)r * nb;
+            for (size_t b = 0; b < nb; b++) {
+                const int E5 = (bs[b] >> 10) & 31, mant = bs[b] & 1023;
+                const uint32_t ms = (uint32_t)(E5 ? 1024 + mant : mant) << ((E5 ? E5 - 25 : -24) + 9 - et[r] < 0 ? 0 : (E5 ? E5 - 25 : -24) + 9 - et[r]);
+                if (ms & 255) exl.push_back((uint32_t)(r & 15) | (uint32_t)b << 4 | (ms & 255) << 24);
+            }
+            if (r % 16 == 15 || r == rows - 1) exo[r / 16 + 1] = (uint32_t)exl.size();
+        }
+        fold = exl.size() <= FOLD_LIST_MAX * (double)rows * (double)nb ? 2 : 3;
+        if (fold == 3) { exl.clear(); std::fill(exo.begin(), exo.end(), 0u); }
     }
     // the GEMV's copy of the scales, il rows interleaved per block
     bs8_store.emplace_back((size_t)(rows + il - 1) / il * il * nb, (uint16_t)0);
@@ -221,7 +242,10 @@ int load_weight(const qwen3_model *qm, const gguf_tensor *t, int rows, int cols,
     offs[1] = up.add(p.bscale, nb * 2 * rows);
     offs[2] = up.add(eb.data(), (size_t)rows + 8);
     offs[3] = up.add(b8.data(), b8.size() * 2);
-    w.rows = rows; w.cols = cols; w.nblk = (int)nb; w.wide = wide; w.il = il;
+    offs[4] = up.add(et.data(), (size_t)rows);
+    offs[5] = up.add(ex_store[ex_store.size() - 2].data(), ex_store[ex_store.size() - 2].size() * 4);
+    offs[6] = up.add(ex_store.back().data(), ex_store.back().size() * 4);
+    w.rows = rows; w.cols = cols; w.nblk = (int)nb; w.wide = wide; w.il = il; w.fold = fold;
     return 0;
 }
 
@@ -260,13 +284,15 @@ DevModel *model_get(const qwen3_model *qm, bool upload = true) {
     Uploader up;
     std::vector<std::vector<int8_t>> ebs;
     std::vector<std::vector<uint16_t>> b8s;
-    ebs.reserve((size_t)m->NL * 7 + 2);
+    ebs.reserve(2 * ((size_t)m->NL * 7 + 2));
     b8s.reserve((size_t)m->NL * 7 + 2);
-    struct Pending { DevW *w; size_t o[4]; };
+    std::vector<std::vector<uint32_t>> exs;
+    exs.reserve(2 * ((size_t)m->NL * 7 + 2));
+    struct Pending { DevW *w; size_t o[7]; };
     std::vector<Pending> pend;
     auto addw = [&](const gguf_tensor *t, int rows, int cols, DevW &w, int il = 8) -> int {
         Pending pd; pd.w = &w;
-        if (load_weight(qm, t, rows, cols, up, ebs, b8s, w, pd.o, il)) return 1;
+        if (load_weight(qm, t, rows, cols, up, ebs, b8s, exs, w, pd.o, il)) return 1;
         pend.push_back(pd);
         return 0;
     };
@@ -341,7 +367,7 @@ DevModel *model_get(const qwen3_model *qm, bool upload = true) {
     }
     uint8_t *base = (uint8_t *)m->buf;
     for (size_t i = 0; i < up.src.size(); i++)
-        if (hipMemcpy(base + up.off[i], up.src[i].first, up.src[i].second, hipMemcpyHostToDevice) != hipSuccess) {
+        if (up.src[i].second && hipMemcpy(base + up.off[i], up.src[i].first, up.src[i].second, hipMemcpyHostToDevice) != hipSuccess) {
             hipFree(m->buf); fail("sp_hipkv_open: weight upload failed%s", ""); return nullptr;
         }
     for (auto &pd : pend) {
@@ -349,6 +375,9 @@ DevModel *model_get(const qwen3_model *qm, bool upload = true) {
         pd.w->bs = (const uint16_t *)(base + pd.o[1]);
         pd.w->ebase = (const int8_t *)(base + pd.o[2]);
         pd.w->bs8 = (const uint16_t *)(base + pd.o[3]);
+        pd.w->etop = (const int8_t *)(base + pd.o[4]);
+        pd.w->exo = (const int *)(base + pd.o[5]);
+        pd.w->exl = (const uint32_t *)(base + pd.o[6]);
     }
     for (size_t i = 0; i < norm_slots.size(); i++) *norm_slots[i] = (const float *)(base + norm_off[i]);
     if (tied) m->out = m->embd;
@@ -1141,7 +1170,9 @@ int run_batch(sp_kvdecode_handle *h, int T, int pos0, int pos_hi, bool multi, Ti
     const DevModel *m = h->m;
     auto &b = h->b;
     hipStream_t s = h->stream;
-    const int QD = m->NH * m->HD, KVD = m->NKV * m->HD, TP = (T + 31) / 32 * 32;
+    const int QD = m->NH * m->HD, KVD = m->NKV * m->HD;
+    // padded tokens of a GEMM: 16-token tiles where every segment folds
+    auto tp = [&](bool fold) { return fold ? (T + 15) / 16 * 16 : (T + 31) / 32 * 32; };
     auto TM = [&](int cls, bool begin) { if (cb) cb(ctx, cls, begin); };
     TM(8, true);
     launch_embed_batch(m->embd, h->tokbuf, pos0, T, b.x1, m->gemma ? sqrtf((float)m->E) : 0.0f, s,
@@ -1151,26 +1182,27 @@ int run_batch(sp_kvdecode_handle *h, int T, int pos0, int pos_hi, bool multi, Ti
                             multi ? b.tpos : nullptr);
     TM(8, false);
     auto stage = [&](int kind, const float *x, const float *delta, const float *post_w, const float *norm_w,
-                     float *x_out, int n) {
+                     float *x_out, int n, bool fold) {
         StageArgs a{};
         a.pro.kind = kind; a.pro.x = x; a.pro.delta = delta; a.pro.post_w = post_w; a.pro.norm_w = norm_w;
         a.pro.x_out = x_out; a.pro.n = n; a.pro.eps = m->eps;
-        a.planes = b.planes; a.sh = b.sh; a.T = T; a.TP = TP; a.mode = h->mode;
+        a.planes = b.planes; a.sh = b.sh; a.T = T; a.TP = tp(fold); a.mode = h->mode; a.fold = fold;
         launch_stage(a, s);
     };
-    auto gemm = [&](int cols) {
+    auto gemm = [&](int cols, bool fold) {
         GemmArgs g{};
-        g.cols = cols; g.planes = b.planes; g.sh = b.sh; g.T = T; g.TP = TP; g.mode = h->mode; g.act = ACT_NONE;
+        g.cols = cols; g.planes = b.planes; g.sh = b.sh; g.T = T; g.TP = tp(fold); g.fold = fold; g.mode = h->mode; g.act = ACT_NONE;
         g.part = b.gpart; g.part_cap = GEMM_PART_BYTES / 8; g.cnt = b.gcnt; g.cnt_cap = GEMM_TILE_COUNTERS;
         return g;
     };
     for (int l = 0; l < m->NL; l++) {
         const DevLayer &d = m->L[l];
         const bool glob = is_global(m, l);
+        const bool fqkv = gemm_folds(d.q) && gemm_folds(d.k) && gemm_folds(d.v);
         TM(0, true);
-        if (l == 0) stage(PRO_NORM, b.x1, nullptr, nullptr, d.attn_norm, nullptr, m->E);
-        else stage(PRO_RESID, b.x0, b.dn, m->gemma ? m->L[l - 1].post_ffw : nullptr, d.attn_norm, b.x1, m->E);
-        GemmArgs g = gemm(m->E);
+        if (l == 0) stage(PRO_NORM, b.x1, nullptr, nullptr, d.attn_norm, nullptr, m->E, fqkv);
+        else stage(PRO_RESID, b.x0, b.dn, m->gemma ? m->L[l - 1].post_ffw : nullptr, d.attn_norm, b.x1, m->E, fqkv);
+        GemmArgs g = gemm(m->E, fqkv);
         g.nseg = 3; g.seg[0] = {d.q, b.q}; g.seg[1] = {d.k, b.k}; g.seg[2] = {d.v, b.v};
         launch_gemm(g, QD + 2 * KVD, s);
         TM(0, false);
@@ -1206,23 +1238,24 @@ int run_batch(sp_kvdecode_handle *h, int T, int pos0, int pos_hi, bool multi, Ti
         TM(a.win >= 0 ? 6 : 5, true); launch_attention(a, nch, s); TM(a.win >= 0 ? 6 : 5, false);
 
         TM(1, true);
-        stage(PRO_PLAIN, b.ao, nullptr, nullptr, nullptr, nullptr, QD);
-        GemmArgs o = gemm(QD);
+        stage(PRO_PLAIN, b.ao, nullptr, nullptr, nullptr, nullptr, QD, gemm_folds(d.o));
+        GemmArgs o = gemm(QD, gemm_folds(d.o));
         o.nseg = 1; o.seg[0] = {d.o, b.ap};
         launch_gemm(o, m->E, s);
         TM(1, false);
 
         TM(2, true);
-        stage(PRO_RESID, b.x1, b.ap, d.post_attn, d.ffn_norm, b.x0, m->E);
-        GemmArgs f = gemm(m->E);
+        const bool fgu = gemm_folds(d.gate) && gemm_folds(d.up);
+        stage(PRO_RESID, b.x1, b.ap, d.post_attn, d.ffn_norm, b.x0, m->E, fgu);
+        GemmArgs f = gemm(m->E, fgu);
         f.nseg = 2; f.act = m->gemma ? ACT_GELU : ACT_SILU;
         f.seg[0] = {d.gate, b.gg}; f.seg[1] = {d.up, b.uu}; f.act_out = b.hh;
         launch_gemm(f, m->FF, s);
         TM(2, false);
 
         TM(3, true);
-        stage(PRO_PLAIN, b.hh, nullptr, nullptr, nullptr, nullptr, m->FF);
-        GemmArgs dd = gemm(m->FF);
+        stage(PRO_PLAIN, b.hh, nullptr, nullptr, nullptr, nullptr, m->FF, gemm_folds(d.down));
+        GemmArgs dd = gemm(m->FF, gemm_folds(d.down));
         dd.nseg = 1; dd.seg[0] = {d.down, b.dn};
         launch_gemm(dd, m->E, s);
         TM(3, false);
@@ -1230,8 +1263,8 @@ int run_batch(sp_kvdecode_handle *h, int T, int pos0, int pos_hi, bool multi, Ti
     if (multi) {
         // LM head over the T rows, then each row's greedy token
         TM(4, true);
-        stage(PRO_RESID, b.x0, b.dn, m->gemma ? m->L[m->NL - 1].post_ffw : nullptr, m->out_norm, nullptr, m->E);
-        GemmArgs lm = gemm(m->E);
+        stage(PRO_RESID, b.x0, b.dn, m->gemma ? m->L[m->NL - 1].post_ffw : nullptr, m->out_norm, nullptr, m->E, gemm_folds(m->out));
+        GemmArgs lm = gemm(m->E, gemm_folds(m->out));
         lm.nseg = 1; lm.seg[0] = {m->out, b.logits};
         launch_gemm(lm, m->V, s);
         launch_argmax_rows(b.logits, m->V, T, b.next, s);

@@ -33,6 +33,14 @@ struct DevW {
     const uint16_t *bs8;
     int rows, cols, nblk, wide;   // wide: a row's exponent spread needs the int128 path
     int il;
+    const int8_t *etop;           // [rows] largest block exponent of the row
+    // the folded GEMM (kvd_gemm.hip): 0 = some block's exponent is more than 9
+    // below its row's etop (or a negative scale); 2 = at most FOLD_LIST_MAX of
+    // the blocks have a low byte, listed per 16-row tile: exl[exo[tile] ..
+    // exo[tile + 1]) = row in tile | block << 4 | low byte << 24; 3 = more do
+    int fold;
+    const int *exo;
+    const uint32_t *exl;
 };
 
 // Whole-vector statistics that the kernel producing a vector accumulates while
@@ -186,7 +194,8 @@ struct StageArgs {
     ProArgs pro;
     int8_t *planes;
     int *sh;           // [TP] grid exponent per token (SH_ZERO: all-zero input)
-    int T, TP, mode;   // tokens, padded token count (multiple of 32)
+    int T, TP, mode;   // tokens, padded token count (multiple of 32; folded: 16)
+    int fold;          // the folded GEMM's operand order (kvd_prefill.hip)
 };
 // OK_Q4B GEMM over T staged tokens: seg[i].out is [T][seg rows]; paired
 // gate/up write gate, up and act(gate)*up ([T][rows]).
@@ -196,6 +205,7 @@ struct GemmArgs {
     const int8_t *planes;
     const int *sh;
     int  T, TP;
+    int  fold;         // planes are in the folded GEMM's order
     int  act;
     float *act_out;
     int  mode;
@@ -268,6 +278,11 @@ void launch_argmax_rows(const float *logits, int V, int T, int *out, hipStream_t
 void launch_stage(const StageArgs &a, hipStream_t s);
 void launch_gemm(const GemmArgs &a, int nrows_total, hipStream_t s);
 bool gemm_supported(const DevW &w);
+// the GEMM with the block scales folded into the weight digits (kvd_gemm.hip),
+// for launches whose segments all fold (TP: a multiple of 16)
+int gemm_folds(const DevW &w);
+constexpr double FOLD_LIST_MAX = 0.02;
+void launch_gemm_fold(const GemmArgs &a, int nrows_total, hipStream_t s);
 void launch_advance(DState *st, hipStream_t s);
 void launch_gemv(const GemvArgs &a, int nrows_total, hipStream_t s);
 void gemv_time_next(hipEvent_t start, hipEvent_t stop);   // events of the calling thread's next GEMV launch

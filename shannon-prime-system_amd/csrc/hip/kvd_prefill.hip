@@ -28,17 +28,27 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 // bytes of a (block, token) follow the A operand's unpack order: within each
 // group of 8 columns 8g..8g+7 the order is 8g + {0, 2, 4, 6, 1, 3, 5, 7}
 // (low nibbles, then high nibbles, of the packed codes).
-template <int PRO>
+// FOLD (kvd_gemm.hip): planes[p][128-column super-step][half m][16-token tile]
+// [lane = 16 g + token % 16][16 bytes]: columns 16 m .. 16 m + 15 of block
+// 4 s + g, each 8 in the order 0 1 4 5 2 3 6 7 -- the MFMA A operand as a wave
+// reads it, 1 KiB per operand.
+template <int PRO, bool FOLD>
 __global__ __launch_bounds__(512) void k_stage(StageArgs a) {
     extern __shared__ float xf[];                      // pro.n floats (norm prologues)
     __shared__ double red[RED_SLOTS * RED_WAVES];
     const int t = blockIdx.x, n = a.pro.n, nblk = n / 32, tid = threadIdx.x;
     int8_t *planes = a.planes;
+    // byte offset of 8-column group g of plane pl for this token
+    auto at = [&](int pl, int g) -> size_t {
+        const int b = g >> 2, q = g & 3;
+        if (FOLD) return ((((size_t)pl * (nblk >> 2) + (b >> 2)) * 2 + (q >> 1)) * (a.TP >> 4) + (t >> 4)) * 1024 +
+                         ((b & 3) * 16 + (t & 15)) * 16 + 8 * (q & 1);
+        return (((size_t)pl * nblk + b) * a.TP + t) * 32 + 8 * q;
+    };
     if (t >= a.T) {                                     // padding tokens: zero planes
         for (int g = tid; g < nblk * 4; g += blockDim.x)
             #pragma unroll
-            for (int p = 0; p < 3; p++)
-                *(uint2 *)(planes + (((size_t)p * nblk + (g >> 2)) * a.TP + t) * 32 + 8 * (g & 3)) = make_uint2(0, 0);
+            for (int p = 0; p < 3; p++) *(uint2 *)(planes + at(p, g)) = make_uint2(0, 0);
         if (tid == 0) a.sh[t] = SH_ZERO;
         return;
     }
@@ -57,7 +67,9 @@ __global__ __launch_bounds__(512) void k_stage(StageArgs a) {
             #pragma unroll
             for (int j = 0; j < 8; j++) {
                 int32_t q = (int32_t)rintf(ldexpf(v[j], sh));
-                const int slot = (j & 1) ? 4 + (j >> 1) : (j >> 1);      // unpack order
+                // unpack order of the codes (folded: 0 1 4 5 2 3 6 7)
+                const int slot = FOLD ? ((j & 2) ? (j & 5) + (j < 4 ? 4 : 2) : (j & 1) + (j < 4 ? 0 : 2))
+                                      : ((j & 1) ? 4 + (j >> 1) : (j >> 1));
                 #pragma unroll
                 for (int pl = 0; pl < 3; pl++) {
                     const int32_t d = ((q + 128) & 255) - 128;
@@ -69,7 +81,7 @@ __global__ __launch_bounds__(512) void k_stage(StageArgs a) {
         }
         #pragma unroll
         for (int pl = 0; pl < 3; pl++)
-            *(uint2 *)(planes + (((size_t)pl * nblk + (g >> 2)) * a.TP + t) * 32 + 8 * (g & 3)) = make_uint2(lo[pl], hi[pl]);
+            *(uint2 *)(planes + at(pl, g)) = make_uint2(lo[pl], hi[pl]);
     }
 }
 
@@ -343,11 +355,17 @@ __global__ __launch_bounds__(256) void k_gemm_q4b(GemmArgs a) {
 // ------------------------------------------------------------- launchers
 void launch_stage(const StageArgs &a, hipStream_t s) {
     const size_t lds = a.pro.kind == PRO_PLAIN ? 0 : (size_t)a.pro.n * sizeof(float);
-    if (a.pro.n % 32 || a.TP % 32 || a.T > a.TP) { launch_fail("GEMM staging shape outside the kernel's limits"); return; }
-    switch (a.pro.kind) {
-    case PRO_PLAIN: hipLaunchKernelGGL(k_stage<PRO_PLAIN>, dim3(a.TP), dim3(512), lds, s, a); break;
-    case PRO_NORM:  hipLaunchKernelGGL(k_stage<PRO_NORM>, dim3(a.TP), dim3(512), lds, s, a); break;
-    default:        hipLaunchKernelGGL(k_stage<PRO_RESID>, dim3(a.TP), dim3(512), lds, s, a); break;
+    if (a.pro.n % (a.fold ? 128 : 32) || a.TP % (a.fold ? 16 : 32) || a.T > a.TP) {
+        launch_fail("GEMM staging shape outside the kernel's limits"); return;
+    }
+    const dim3 grid(a.TP), wg(512);
+    switch (a.pro.kind * 2 + (a.fold ? 1 : 0)) {
+    case PRO_PLAIN * 2:     hipLaunchKernelGGL((k_stage<PRO_PLAIN, false>), grid, wg, lds, s, a); break;
+    case PRO_PLAIN * 2 + 1: hipLaunchKernelGGL((k_stage<PRO_PLAIN, true>), grid, wg, lds, s, a); break;
+    case PRO_NORM * 2:      hipLaunchKernelGGL((k_stage<PRO_NORM, false>), grid, wg, lds, s, a); break;
+    case PRO_NORM * 2 + 1:  hipLaunchKernelGGL((k_stage<PRO_NORM, true>), grid, wg, lds, s, a); break;
+    case PRO_RESID * 2:     hipLaunchKernelGGL((k_stage<PRO_RESID, false>), grid, wg, lds, s, a); break;
+    default:                hipLaunchKernelGGL((k_stage<PRO_RESID, true>), grid, wg, lds, s, a); break;
     }
 }
 
@@ -361,6 +379,11 @@ void launch_gemm(const GemmArgs &a, int nrows_total, hipStream_t s) {
         if (!gemm_supported(a.seg[i].w) || a.seg[i].w.cols != a.cols) {
             launch_fail("GEMM segment shape not supported"); return;
         }
+    if (a.fold) {
+        for (int i = 0; i < a.nseg; i++)
+            if (!gemm_folds(a.seg[i].w)) { launch_fail("GEMM segment does not fold"); return; }
+        return launch_gemm_fold(a, nrows_total, s);
+    }
     if (nrows_total % 64 || a.TP % 32 || a.T > a.TP) { launch_fail("GEMM rows or token count outside the kernel's limits"); return; }
     // the kernel's buffer offsets are 32-bit: planes (3 x nblk x TP x 32 bytes)
     // and one 16-row slice of codes / scales

@@ -136,3 +136,28 @@ def oracle_ppl(o, toks, n_warm):
         nll += -(float(lg[tgt]) - maxl - math.log(se))
         ns += 1
     return math.exp(nll / ns)
+
+
+def write_scaled(dirpath, name, share, down):
+    """The SMALL model `name` with a seeded `share` of every matrix's 32-column
+    block scales multiplied by 2^-down in the file (exact in f16 down to its
+    smallest step): returns the paths and the shape."""
+    d = SMALL[name]
+    prefix = os.path.join(str(dirpath), f"{name}_x{share}_{down}")
+    spm, spt = prefix + ".spm", prefix + ".spt"
+    if not os.path.exists(spm):
+        spkv.write_model(prefix, max_context=512, **d)
+        raw = np.memmap(spm, dtype=np.uint8, mode="r+")
+        count = int(raw[316:320].view(np.uint32)[0])
+        table, data = (int(x) for x in raw[320:336].view(np.uint64))
+        rng = np.random.default_rng(5)
+        for i in range(count):
+            e = raw[table + 256 * i:table + 256 * (i + 1)]
+            if bytes(e[:80]).split(b"\0")[0].endswith(b".bscale") and share:
+                off, size = (int(x) for x in e[152:168].copy().view(np.uint64))
+                sc = raw[data + off:data + off + size].view(np.float16)
+                pick = rng.random(sc.size) < share
+                sc[pick] = (sc[pick].astype(np.float32) * np.float32(2.0 ** -down)).astype(np.float16)
+        raw.flush()
+        del raw
+    return spm, spt, d
