@@ -455,7 +455,7 @@ __global__ __launch_bounds__(64 * FOLD_WAVES, 2) void k_gemm_fold(GemmArgs a) {
             #pragma unroll
             for (int r = 0; r < RT; r++) {
                 y[r] = sh == SH_ZERO ? 0.0f : rne_scaled(tot[r][j][i], top[r] - 9 - sh);
-                if (live[r]) a.seg[seg[r]].out[(size_t)t * a.seg[seg[r]].w.rows + rb0[r] + n16] = y[r];
+                if (!PAIRED && live[r]) a.seg[seg[r]].out[(size_t)t * a.seg[seg[r]].w.rows + rb0[r] + n16] = y[r];
             }
             if constexpr (PAIRED)
                 if (live[0]) a.act_out[(size_t)t * a.seg[0].w.rows + rb0[0] + n16] = act_apply(y[0], y[1], a.act, a.mode);

@@ -198,7 +198,7 @@ struct StageArgs {
     int fold;          // the folded GEMM's operand order (kvd_prefill.hip)
 };
 // OK_Q4B GEMM over T staged tokens: seg[i].out is [T][seg rows]; paired
-// gate/up write gate, up and act(gate)*up ([T][rows]).
+// gate/up write act(gate)*up only (act_out, [T][rows]).
 struct GemmArgs {
     Seg  seg[3];
     int  nseg, cols;

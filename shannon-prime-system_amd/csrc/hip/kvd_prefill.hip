@@ -344,7 +344,6 @@ __global__ __launch_bounds__(256) void k_gemm_q4b(GemmArgs a) {
             if (PAIRED) {
                 const float yb = sh == SH_ZERO ? 0.0f : rne_i64_scaled(acc_b[j][i], eb_b - sh);
                 const size_t o = (size_t)t * wa.rows + row;
-                a.seg[0].out[o] = ya; a.seg[1].out[o] = yb;
                 a.act_out[o] = act_apply(ya, yb, a.act, a.mode);
             } else {
                 a.seg[s].out[(size_t)t * wa.rows + row] = ya;
