@@ -13,24 +13,45 @@ typedef unsigned __int128 u128;
 constexpr int FB = 30;
 constexpr int64_t ONE = (int64_t)1 << FB;
 constexpr int64_t LOG2E = 1549082005LL;                    // round(log2(e) * 2^30)
-__device__ constexpr int64_t EXPC[7] = {1073741824LL, 744261118LL, 257941248LL, 59597083LL,
+static constexpr int64_t EXPC[7] = {1073741824LL, 744261118LL, 257941248LL, 59597083LL,
                                         10327387LL, 1431680LL, 165394LL};   // round((ln2)^k/k! * 2^30)
 constexpr int64_t GK = 856722024LL;                        // round(sqrt(2/pi) * 2^30)
 constexpr int64_t GA = 48012366LL;                         // round(0.044715 * 2^30)
 
-__device__ __forceinline__ int64_t exp2_frac(int64_t r) {
-    int64_t acc = EXPC[6];
+// 0 <= r <= 2^30: every partial sum is below 2^31, so each product is one
+// 32 x 32 -> 64 bit multiply
+__host__ __device__ __forceinline__ uint32_t exp2_frac(uint32_t r) {
+    uint32_t acc = (uint32_t)EXPC[6];
     #pragma unroll
-    for (int k = 5; k >= 0; k--) acc = ((acc * r) >> FB) + EXPC[k];
+    for (int k = 5; k >= 0; k--) acc = (uint32_t)(((uint64_t)acc * r) >> FB) + (uint32_t)EXPC[k];
     return acc;
 }
-// e^d for d <= 0, Q30 in and out
-__device__ __forceinline__ int64_t exp_fixed(int64_t d) {
-    int64_t g = (int64_t)(-(((i128)d * LOG2E) >> FB));
-    int64_t n = g >> FB, r = g - (n << FB);
+// e^d for d <= 0, Q30 in and out: 2^-g, g = ceil(-d LOG2E / 2^30) in Q30.
+// From 2^35 on n >= 46 (from 2^62 on the island's 64-bit g wraps, and its steps
+// are kept); below, with -d = 32 a + b, -d LOG2E = 32 u + c,
+// u = a LOG2E + (b LOG2E >> 5) < 2^62, and g = ceil(32 u + c over 2^30)
+__host__ __device__ __forceinline__ int64_t exp_fixed(int64_t d) {
+    const uint64_t D = 0 - (uint64_t)d;
+    if (D >> 62) {
+        const int64_t g = (int64_t)(-(((i128)d * LOG2E) >> FB));
+        const int64_t n = g >> FB, r = g - (n << FB);
+        if (n >= 32) return 0;
+        if (r) return (int64_t)exp2_frac((uint32_t)(ONE - r)) >> (n + 1);
+        return ONE >> n;
+    }
+    if (D >> 35) return 0;
+    const uint32_t bl = (uint32_t)D & 31;
+    const uint64_t bL = (uint64_t)bl * (uint32_t)LOG2E;
+    const uint64_t u = (uint64_t)(uint32_t)(D >> 5) * (uint32_t)LOG2E + (bL >> 5);
+    const uint64_t g = (u >> 25) + (((u & 0x1FFFFFF) | (bL & 31)) != 0);
+    const uint32_t n = (uint32_t)(g >> FB), r = (uint32_t)g & (uint32_t)(ONE - 1);
     if (n >= 32) return 0;
-    if (r) return exp2_frac(ONE - r) >> (n + 1);
+    if (r) return (int64_t)((uint64_t)exp2_frac((uint32_t)ONE - r) >> (n + 1));
     return ONE >> n;
+}
+// (int64_t)(((i128)c * v) >> 30) for 0 <= c < 2^32, any v (the same wrapped value)
+__host__ __device__ __forceinline__ int64_t mul_q30(uint32_t c, int64_t v) {
+    return (int64_t)((uint64_t)c * (uint64_t)(v >> 32) * 4 + (((uint64_t)c * (uint32_t)v) >> 30));
 }
 // floor(sqrt(v)): double estimate, then exact integer correction (the result
 // is the unique floor, identical to the bit-serial isqrt of the islands)
@@ -126,8 +147,20 @@ template <int SH> __device__ __forceinline__ int64_t llround_pow2(float x) {
     return llround_d((double)x * (double)(1 << SH));
 }
 
+// The islands' activations.  With |xq| below the bounds (|x| < 16 and |x| < 2^15)
+// X = xq 2^14 is taken apart, so that every product of the 128-bit form is a
+// 64-bit one or two with the same floor: X^2 >> 30 = xq^2 >> 2, and so on.  A
+// gate/up epilogue of the batched GEMM spent as long on the 128-bit form as on a
+// quarter of its products.
 __device__ __forceinline__ float gelu_exact1(float x) {
     int64_t xq = llround_pow2<16>(x);
+    if (xq > -(1 << 20) && xq < (1 << 20)) {
+        const int32_t q = (int32_t)xq;
+        const int64_t x2 = ((int64_t)q * q) >> 2;                   // below 2^38
+        const int64_t x3 = (x2 * q) >> 16;
+        const int64_t t = tanh_fixed(mul_q30((uint32_t)GK, ((int64_t)q << 14) + mul_q30((uint32_t)GA, x3)));
+        return (float)((double)(((int64_t)q * (ONE + t)) >> 17) * 0x1p-30);   // (X >> 1)(ONE + t) >> 30
+    }
     int64_t X = (xq * ONE) >> 16;
     i128 X2 = ((i128)X * X) >> FB;
     int64_t x3 = (int64_t)((X2 * X) >> FB);
@@ -138,6 +171,11 @@ __device__ __forceinline__ float gelu_exact1(float x) {
 }
 __device__ __forceinline__ float silu_exact1(float x) {
     int64_t xq = llround_pow2<16>(x);
+    if (xq > -((int64_t)1 << 31) && xq < ((int64_t)1 << 31)) {
+        const int64_t X = xq << 14, e = exp_fixed(X >= 0 ? -X : X);
+        const int64_t sg = udiv_small(X >= 0 ? ONE << FB : e << FB, ONE + e);
+        return (float)((double)((xq * sg) >> 16) * 0x1p-30);        // X sg >> 30
+    }
     int64_t X = (xq * ONE) >> 16;
     int64_t e = exp_fixed(X >= 0 ? -X : X);
     int64_t sg = X >= 0 ? udiv_small(ONE << FB, ONE + e)          // 2^60 / [2^30, 2^31]
@@ -175,7 +213,11 @@ __device__ __forceinline__ float rne_u128_scaled(u128 mag, int k) {
 __device__ __forceinline__ float rne_i128_scaled(i128 v, int k) {
     return v >= 0 ? rne_u128_scaled((u128)v, k) : -rne_u128_scaled((u128)(-v), k);
 }
+// the conversion rounds to nearest even and the scaling is exact where the
+// result is a normal float; the general path takes the rest
 __device__ __forceinline__ float rne_i64_scaled(int64_t v, int k) {
+    const float f = ldexpf((float)v, k), m = fabsf(f);
+    if (m >= 0x1p-126f && m < INFINITY) return f;
     return v >= 0 ? rne_u128_scaled((u128)(uint64_t)v, k) : -rne_u128_scaled((u128)(uint64_t)(-v), k);
 }
 // RNE of num / (den * 2^k), den > 0

@@ -113,14 +113,6 @@ constexpr int fold_depth(int WK, int TT) {
     return d < 6 ? d : 6;
 }
 
-// RNE of v 2^k: the hardware's int64 -> float rounding (nearest even) and an
-// exact scaling where the result is a normal float, else the general path
-__device__ __forceinline__ float rne_scaled(int64_t v, int k) {
-    const float r = ldexpf((float)v, k);
-    const float m = fabsf(r);
-    return (m >= 1.17549435e-38f && m < INFINITY) || v == 0 ? r : rne_i64_scaled(v, k);
-}
-
 }  // namespace
 
 // A workgroup's 8 waves are WR = 8 / WK row groups x WK K groups; it owns TT
@@ -383,46 +375,40 @@ __global__ __launch_bounds__(64 * FOLD_WAVES, 2) void k_gemm_fold(GemmArgs a) {
             }
         }
     }
-    // K groups meet: token tile j is finished by K group j % WK, which adds the
-    // others' sums from LDS [(K group, row group, tile r, j, i)][lane]
-    if constexpr (WK > 1) {
-        static_assert(FOLD_WAVES * RT * TT * 4 * 64 * 8 <= LDS, "the K groups' sums fit the ring");
-        int64_t *ex = (int64_t *)ring;
-        auto at = [&](int k, int r, int j, int i) { return ((((k * WR + wr) * RT + r) * TT + j) * 4 + i) * 64 + lane; };
+    // The sums go through LDS, [(K group, row group, tile r, j, i)][lane]: the K
+    // groups meet there, each finishing every WK-th (j, i), in loops that stay
+    // rolled (unrolled, the rounding and the activation of 32 outputs per lane
+    // are more code than the rest).
+    constexpr int ITEMS = TT * 4;
+    static_assert(FOLD_WAVES * RT * ITEMS * 64 * 8 <= LDS, "the sums fit the rings");
+    int64_t *const ex = (int64_t *)ring + lane;
+    auto at = [&](int k, int r, int it) { return (((k * WR + wr) * RT + r) * ITEMS + it) * 64; };
+    #pragma unroll
+    for (int r = 0; r < RT; r++)
         #pragma unroll
-        for (int r = 0; r < RT; r++)
-            #pragma unroll
-            for (int j = 0; j < TT; j++)
-                #pragma unroll
-                for (int i = 0; i < 4; i++) if (j % WK != kg) ex[at(kg, r, j, i)] = tot[r][j][i];
-        __syncthreads();
+        for (int it = 0; it < ITEMS; it++) ex[at(kg, r, it)] = tot[r][it >> 2][it & 3];
+    __syncthreads();
+    auto sum_of = [&](int r, int it) {
+        int64_t v = 0;
         #pragma unroll
-        for (int r = 0; r < RT; r++)
-            #pragma unroll
-            for (int j = 0; j < TT; j++)
-                #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (j % WK == kg)
-                        for (int k = 0; k < WK; k++) if (k != kg) tot[r][j][i] += ex[at(k, r, j, i)];
-    }
-    auto mine = [&](int j) { return WK == 1 || j % WK == kg; };
-    const int t0 = tile0 * 16 + 4 * g;                 // lane's tokens: t0 + 16 j + i
+        for (int k = 0; k < WK; k++) v += ex[at(k, r, it)];
+        return v;
+    };
+    const int t0 = tile0 * 16 + 4 * g;                 // lane's tokens: t0 + 16 (it / 4) + it % 4
+    // where a split keeps its partial of (r, token t)
+    auto slot = [&](int r, int t) { return (size_t)t * a.arows + (PAIRED && r ? a.arows / 2 : 0) + grow[r] + n16; };
+    const size_t zs = (size_t)a.TP * a.arows;
     if constexpr (SPLIT) {
         // every split stores its exact partials in its own slice (agent-scope
         // stores, coherent across the XCDs' L2s); the tile's last split adds
         // the others' to its own
-        const size_t zs = (size_t)a.TP * a.arows;
-        auto at = [&](int r, int j, int i) {
-            return (size_t)(t0 + 16 * j + i) * a.arows + (PAIRED && r ? a.arows / 2 : 0) + grow[r] + n16;
-        };
-        int64_t *own = a.part + blockIdx.z * zs;
-        #pragma unroll
-        for (int r = 0; r < RT; r++)
+        #pragma unroll 1
+        for (int it = kg; it < ITEMS; it += WK) {
+            const int t = t0 + 16 * (it >> 2) + (it & 3);
             #pragma unroll
-            for (int j = 0; j < TT; j++)
-                #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (mine(j) && live[r] && tile0 + j < NT) st_agent(&own[at(r, j, i)], tot[r][j][i]);
+            for (int r = 0; r < RT; r++)
+                if (live[r] && t < a.TP) st_agent(&a.part[blockIdx.z * zs + slot(r, t)], sum_of(r, it));
+        }
         mem_complete();
         __shared__ int last;
         __syncthreads();
@@ -430,36 +416,25 @@ __global__ __launch_bounds__(64 * FOLD_WAVES, 2) void k_gemm_fold(GemmArgs a) {
         if (tid == 0) last = arrive(cnt) == (int)gridDim.z - 1;
         __syncthreads();
         if (!last) return;
-        for (int z = 0; z < (int)gridDim.z; z++) {
-            if (z == (int)blockIdx.z) continue;
-            const int64_t *other = a.part + z * zs;
-            #pragma unroll
-            for (int r = 0; r < RT; r++)
-                #pragma unroll
-                for (int j = 0; j < TT; j++)
-                    #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        if (mine(j) && tile0 + j < NT) tot[r][j][i] += ld_agent(&other[at(r, j, i)]);
-        }
         if (tid == 0) reset_counter(cnt);
     }
-    #pragma unroll
-    for (int j = 0; j < TT; j++) {
-        if (!mine(j)) continue;
+    #pragma unroll 1
+    for (int it = kg; it < ITEMS; it += WK) {
+        const int t = t0 + 16 * (it >> 2) + (it & 3);
+        if (t >= a.T) continue;
+        const int sh = a.sh[t];
+        float y[RT];
         #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int t = t0 + 16 * j + i;
-            if (t >= a.T) continue;
-            const int sh = a.sh[t];
-            float y[RT];
-            #pragma unroll
-            for (int r = 0; r < RT; r++) {
-                y[r] = sh == SH_ZERO ? 0.0f : rne_scaled(tot[r][j][i], top[r] - 9 - sh);
-                if (!PAIRED && live[r]) a.seg[seg[r]].out[(size_t)t * a.seg[seg[r]].w.rows + rb0[r] + n16] = y[r];
-            }
-            if constexpr (PAIRED)
-                if (live[0]) a.act_out[(size_t)t * a.seg[0].w.rows + rb0[0] + n16] = act_apply(y[0], y[1], a.act, a.mode);
+        for (int r = 0; r < RT; r++) {
+            int64_t v = sum_of(r, it);
+            if constexpr (SPLIT)
+                for (int z = 0; z < (int)gridDim.z; z++)
+                    if (z != (int)blockIdx.z) v += ld_agent(&a.part[z * zs + slot(r, t)]);
+            y[r] = sh == SH_ZERO ? 0.0f : rne_i64_scaled(v, top[r] - 9 - sh);
+            if (!PAIRED && live[r]) a.seg[seg[r]].out[(size_t)t * a.seg[seg[r]].w.rows + rb0[r] + n16] = y[r];
         }
+        if constexpr (PAIRED)
+            if (live[0]) a.act_out[(size_t)t * a.seg[0].w.rows + rb0[0] + n16] = act_apply(y[0], y[1], a.act, a.mode);
     }
 }
 
