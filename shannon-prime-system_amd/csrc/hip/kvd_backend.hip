@@ -1239,7 +1239,9 @@ int run_batch(sp_kvdecode_handle *h, int T, int pos0, int pos_hi, bool multi, Ti
         // chunks of the batch's longest span: a window of W positions covers at
         // most (W-1)/chunk + 2 chunks whatever its alignment
         TM(a.win >= 0 ? 6 : 5, true);
-        for (int t = 0; t < T; t += b.TB) {                     // one pass for a batched decode
+        if (!multi) a.part_tokens = b.TB;
+        if (prefill_attention_float(a)) launch_prefill_float(a, s);
+        else for (int t = 0; t < T; t += b.TB) {                // one pass for a batched decode
             AttnArgs c = a;
             c.q += (size_t)t * QD; c.k += (size_t)t * KVD; c.v += (size_t)t * KVD; c.qr += (size_t)t * QD; c.ao += (size_t)t * QD;
             c.rope_cs += (size_t)t * c.rope_stride;

@@ -111,6 +111,7 @@ struct AttnArgs {
     // batched prefill: nt tokens at positions pos0.. (token = blockIdx.y of
     // qk_prep, blockIdx.z of attention); every per-token buffer is [nt][...]
     int nt, pos0, rope_stride;
+    int part_tokens;         // float prefill: tokens the part / part_ml buffers hold at max_chunks each (0: the per-token kernels)
     // batched decode over several sessions: token t's position and this
     // layer's page table (NULL: pos0 + t and `pages`)
     const int *tpos;
@@ -165,6 +166,9 @@ void launch_recall_attention(const RecallArgs &rc, hipStream_t s);
 // (token-shared K/V reads, the score pass on the int8 matrix cores)
 bool prefill_attention_tiled(const AttnArgs &a);
 void launch_prefill_attention(const AttnArgs &a, hipStream_t s);
+// ... and float-mode attention of a prefill pass, any number of tokens (kvd_pfloat.hip)
+bool prefill_attention_float(const AttnArgs &a);
+void launch_prefill_float(const AttnArgs &a, hipStream_t s);
 constexpr int RECALL_CHUNK = 64;        // recalled positions per attention workgroup
 constexpr int RECALL_SCORE_BLOCKS = 64; // router scoring workgroups per kv head (grid-stride)
 constexpr int RECALL_MAX_GROUP = 8;     // q heads per kv head the router serves
