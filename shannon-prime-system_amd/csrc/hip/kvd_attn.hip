@@ -287,7 +287,6 @@ __global__ __launch_bounds__(256) void k_attn_float(AttnArgs a_in) {
     __shared__ float sc[G][MAXCH + UNR];             // 0 past the chunk (plain rows' V-sum)
     __shared__ float ored[4][G][EPL * 64];
     __shared__ float wk[MAXNCH];
-    __shared__ float redf[4];
     __shared__ int is_last;
     __shared__ float4 qs[G][EPL * 16];
     for (int i = threadIdx.x; i < G * HD / 4; i += 256) {
@@ -490,35 +489,54 @@ __global__ __launch_bounds__(256) void k_attn_float(AttnArgs a_in) {
     if (threadIdx.x == 0) is_last = (arrive(&a.counter[h]) == nch - 1);
     __syncthreads();
     if (!is_last) return;
+    // The merge is a chain of device-scope round trips, so all heads go at once
+    // (one at a time where their weights don't fit wk): wave k forms head k's
+    // chunk weights, then every thread sums its outputs with 16 partials in
+    // flight.  One head after the other with 4 in flight, the merge was two
+    // thirds of the kernel at 4 096 positions of the Qwen3-0.6B shape (26.2 ->
+    // 17 us).  The sums' order is the same.
     StatAcc sacc;
-    for (int g = 0; g < G; g++) {
-        const size_t base = (size_t)(h * G + g) * a.max_chunks;
-        const float *pml = a.part_ml + base * 2;
-        float mv = -INFINITY;
-        for (int k = threadIdx.x; k < nch; k += 256) mv = fmaxf(mv, ld_agent(&pml[k * 2]));
-        mv = wmax(mv);
-        if (lane == 0) redf[wave] = mv;
-        __syncthreads();
-        const float M = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
-        __syncthreads();
-        float lv = 0.0f;
-        for (int k = threadIdx.x; k < nch; k += 256) { const float w = expf(ld_agent(&pml[k * 2]) - M); wk[k] = w; lv += ld_agent(&pml[k * 2 + 1]) * w; }
-        lv = wsum(lv);
-        if (lane == 0) redf[wave] = lv;
-        __syncthreads();
-        const float L = redf[0] + redf[1] + redf[2] + redf[3];
-        const float *po = a.part + base * HD;
-        for (int d = threadIdx.x; d < HD; d += 256) {
-            float acc0 = 0.0f, acc1 = 0.0f, acc2 = 0.0f, acc3 = 0.0f;
-            int k = 0;
-            for (; k + 4 <= nch; k += 4) {
-                acc0 += ld_agent(&po[(size_t)k * HD + d]) * wk[k];
-                acc1 += ld_agent(&po[(size_t)(k + 1) * HD + d]) * wk[k + 1];
-                acc2 += ld_agent(&po[(size_t)(k + 2) * HD + d]) * wk[k + 2];
-                acc3 += ld_agent(&po[(size_t)(k + 3) * HD + d]) * wk[k + 3];
+    __shared__ float sL[G];
+    const int ng = nch <= MAXNCH / G ? G : 1;
+    for (int g0 = 0; g0 < G; g0 += ng) {
+        if (wave < ng) {
+            const float *pml = a.part_ml + (size_t)(h * G + g0 + wave) * a.max_chunks * 2;
+            float *w_of = wk + wave * (MAXNCH / G);
+            float mv = -INFINITY;
+            for (int k = lane; k < nch; k += 64) mv = fmaxf(mv, ld_agent(&pml[k * 2]));
+            const float M = wmax(mv);
+            float lw[4];
+            #pragma unroll
+            for (int q = 0; q < 4; q++) {
+                float lv = 0.0f;
+                for (int k = lane + 64 * q; k < nch; k += 256) {
+                    const float w = expf(ld_agent(&pml[k * 2]) - M);
+                    w_of[k] = w;
+                    lv += ld_agent(&pml[k * 2 + 1]) * w;
+                }
+                lw[q] = wsum(lv);
             }
-            for (; k < nch; k++) acc0 += ld_agent(&po[(size_t)k * HD + d]) * wk[k];
-            const float o = ((acc0 + acc1) + (acc2 + acc3)) / L;
+            if (lane == 0) sL[g0 + wave] = lw[0] + lw[1] + lw[2] + lw[3];
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < ng * HD; i += 256) {
+            const int gl = i / HD, g = g0 + gl, d = i % HD;
+            const float *po = a.part + (size_t)(h * G + g) * a.max_chunks * HD + d, *w_of = wk + gl * (MAXNCH / G);
+            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            int k = 0;
+            for (; k + 16 <= nch; k += 16) {
+                float x[16];
+                #pragma unroll
+                for (int q = 0; q < 16; q++) x[q] = ld_agent(&po[(size_t)(k + q) * HD]);
+                #pragma unroll
+                for (int q = 0; q < 16; q++) acc[q & 3] += x[q] * w_of[k + q];
+            }
+            for (; k + 4 <= nch; k += 4) {
+                #pragma unroll
+                for (int q = 0; q < 4; q++) acc[q] += ld_agent(&po[(size_t)(k + q) * HD]) * w_of[k + q];
+            }
+            for (; k < nch; k++) acc[0] += ld_agent(&po[(size_t)k * HD]) * w_of[k];
+            const float o = ((acc[0] + acc[1]) + (acc[2] + acc[3])) / sL[g];
             a.ao[(size_t)(h * G + g) * HD + d] = o;
             sacc.add(o);
         }
