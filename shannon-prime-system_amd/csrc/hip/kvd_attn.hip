@@ -155,18 +155,6 @@ __device__ __forceinline__ void rope_table_body(int t_idx, const DState *st, int
         out[(size_t)t * HD + half + i] = s;
     }
 }
-__global__ __launch_bounds__(256) void k_rope_table(const DState *st, int pos0, const int *tpos, int HD, int mode,
-                                                     const int64_t *fq_g, const int64_t *fq_l, float *out) {
-    rope_table_body((int)blockIdx.x, st, pos0, tpos, HD, mode, fq_g, fq_l, out);
-}
-void launch_rope_table(const DState *st, int HD, int mode, float base_g, float base_l,
-                       const int64_t *fq_g, const int64_t *fq_l, float *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_rope_table, dim3(1), dim3(256), 0, s, st, 0, nullptr, HD, mode, fq_g, fq_l, out);
-}
-void launch_rope_table_batch(int pos0, int T, int HD, int mode, float base_g, float base_l,
-                             const int64_t *fq_g, const int64_t *fq_l, float *out, hipStream_t s, const int *tpos) {
-    hipLaunchKernelGGL(k_rope_table, dim3(T), dim3(256), 0, s, nullptr, pos0, tpos, HD, mode, fq_g, fq_l, out);
-}
 void launch_qk_prep(const AttnArgs &a, hipStream_t s) {
     if (a.nt) hipLaunchKernelGGL(k_qk_prep<true>, dim3(a.NH + 2 * a.NKV, a.nt), dim3(64), 0, s, a);
     else hipLaunchKernelGGL(k_qk_prep<false>, dim3(a.NH + 2 * a.NKV), dim3(64), 0, s, a);
@@ -1298,30 +1286,24 @@ __device__ __forceinline__ void embed_body(int t_idx, DevW w, const DState *st, 
         }
     }
 }
-__global__ __launch_bounds__(256) void k_embed(DevW w, const DState *st, const int *tokbuf, int pos0, const int *toks,
-                                                float *x, float scale, VecStat *stats, int nstats) {
-    embed_body((int)blockIdx.x, w, st, tokbuf, pos0, toks, x, scale, stats, nstats);
-}
-// decode: the step's embedding (workgroup 0) and its rotation tables
-// (workgroup 1, independent of it) in one launch
-__global__ __launch_bounds__(256) void k_embed_rope(DevW w, const DState *st, const int *tokbuf, float *x, float scale,
-                                                     VecStat *stats, int nstats, int HD, int mode, const int64_t *fq_g,
-                                                     const int64_t *fq_l, float *rope) {
-    if (blockIdx.x == 0) embed_body(0, w, st, tokbuf, 0, nullptr, x, scale, stats, nstats);
-    else rope_table_body(0, st, 0, nullptr, HD, mode, fq_g, fq_l, rope);
-}
-void launch_embed(const DevW &embd, const DState *st, const int *tokbuf, float *x, float scale, hipStream_t s,
-                  VecStat *stats, int nstats) {
-    hipLaunchKernelGGL(k_embed, dim3(1), dim3(256), 0, s, embd, st, tokbuf, 0, nullptr, x, scale, stats, nstats);
+// The embedding (blockIdx.y = 0) and the rotation tables (1, independent of it)
+// of token blockIdx.x in one launch: a decode step's token (st), or a batch's
+// tokens (their positions pos0 + t or tpos[t]).
+__global__ __launch_bounds__(256) void k_embed_rope(DevW w, const DState *st, const int *tokbuf, int pos0, const int *toks,
+                                                     const int *tpos, float *x, float scale, VecStat *stats, int nstats,
+                                                     int HD, int mode, const int64_t *fq_g, const int64_t *fq_l, float *rope) {
+    if (blockIdx.y == 0) embed_body((int)blockIdx.x, w, st, tokbuf, pos0, toks, x, scale, stats, nstats);
+    else rope_table_body((int)blockIdx.x, st, pos0, tpos, HD, mode, fq_g, fq_l, rope);
 }
 void launch_embed_rope(const DevW &embd, const DState *st, const int *tokbuf, float *x, float scale, VecStat *stats,
                        int nstats, int HD, int mode, const int64_t *fq_g, const int64_t *fq_l, float *rope, hipStream_t s) {
-    hipLaunchKernelGGL(k_embed_rope, dim3(2), dim3(256), 0, s, embd, st, tokbuf, x, scale, stats, nstats, HD, mode,
-                       fq_g, fq_l, rope);
+    hipLaunchKernelGGL(k_embed_rope, dim3(1, 2), dim3(256), 0, s, embd, st, tokbuf, 0, nullptr, nullptr, x, scale, stats, nstats,
+                       HD, mode, fq_g, fq_l, rope);
 }
-void launch_embed_batch(const DevW &embd, const int *tokbuf, int pos0, int T, float *x, float scale, hipStream_t s,
-                        const int *toks) {
-    hipLaunchKernelGGL(k_embed, dim3(T), dim3(256), 0, s, embd, nullptr, tokbuf, pos0, toks, x, scale, nullptr, 0);
+void launch_embed_rope_batch(const DevW &embd, const int *tokbuf, int pos0, const int *toks, const int *tpos, int T, float *x,
+                             float scale, int HD, int mode, const int64_t *fq_g, const int64_t *fq_l, float *rope, hipStream_t s) {
+    hipLaunchKernelGGL(k_embed_rope, dim3(T, 2), dim3(256), 0, s, embd, nullptr, tokbuf, pos0, toks, tpos, x, scale, nullptr, 0,
+                       HD, mode, fq_g, fq_l, rope);
 }
 __global__ void k_advance(DState *st) {
     if (threadIdx.x == 0 && st->drive == DRIVE_STREAM) st->pos = st->pos + 1;

@@ -144,6 +144,41 @@ struct DevLayer {
     DevW q, k, v, o, gate, up, down;
     const float *attn_norm, *q_norm, *k_norm, *ffn_norm, *post_attn, *post_ffw;
 };
+// logits of a batched step leave through pinned slots (logits_to_host)
+constexpr int LOGIT_SLOTS = 4;
+constexpr size_t LOGIT_SLOT_BYTES = (size_t)1 << 20;
+
+// Buffers of the batched calls (prefill, batched decode): [tokens][...] rows, GEMM
+// operands, score grids.  A call leases one from its model and gives it back when
+// its stream has drained (BatchLease), so sessions that prefill one after the
+// other share one, and threads that run at once have one each.
+struct Batch {
+    int mode = 0, pmax = 0;              // its sizes serve this pmax and below; FLOAT's serve both modes
+    void *buf = nullptr;
+    int TB = 0, mcb = 0;                 // tokens per attention batch, chunk capacity per q-head
+    float *x0, *x1, *q, *k, *v, *qr, *ao, *ap, *hh, *dn, *rope, *part, *part_ml;
+    int8_t *planes; int *sh, *counter, *zs;
+    int64_t *vacc, *vacc_s;
+    int64_t *gpart; int *gcnt;           // GEMM split-K partial slices and tile arrival counters
+    // batched decode over sessions (allocated on first use): logits rows,
+    // greedy tokens, per-token token / position / per-layer page tables
+    void *dbuf = nullptr;
+    float *logits; int *next, *toks, *tpos; float *const **tpages;
+    int2 *work; int nwork = 0, wcap = 0;   // full-context layers' (token, chunk) work items
+    void *hstage = nullptr;              // pinned: toks/tpos/tpages/work as uploaded, then:
+    int *hnext = nullptr;                // the greedy tokens
+    uint8_t *hslots = nullptr;           // LOGIT_SLOTS pieces of logits on their way to the caller
+    hipEvent_t slot_ev[LOGIT_SLOTS] = {};
+    void release() {
+        if (buf) hipFree(buf);
+        if (dbuf) hipFree(dbuf);
+        if (hstage) hipHostFree(hstage);
+        for (hipEvent_t e : slot_ev) if (e) hipEventDestroy(e);
+        *this = Batch{};
+    }
+};
+constexpr size_t MAX_IDLE_BATCHES = 4;       // kept by a model; more go back to the device at once
+
 struct DevModel {
     const qwen3_model *qm = nullptr;
     int refs = 0, gemma = 0;
@@ -159,6 +194,8 @@ struct DevModel {
     // captured graphs intact): a fork or open with the same pmax and window ring
     // takes one instead of allocating; they hold no model reference
     std::vector<sp_kvdecode_handle *> shells;
+    std::mutex batch_mu;
+    std::vector<Batch> batches;               // idle, whole (every counter and total at zero)
 };
 std::map<const qwen3_model *, DevModel *> g_models;
 void free_handle(sp_kvdecode_handle *h);
@@ -399,6 +436,7 @@ void model_put(DevModel *m) {
     if (!m || --m->refs > 0) return;
     for (sp_kvdecode_handle *sh : m->shells) free_handle(sh);
     m->shells.clear();
+    for (Batch &b : m->batches) b.release();
     g_models.erase(m->qm);
     hipFree(m->buf);
     delete m;
@@ -549,21 +587,7 @@ struct sp_kvdecode_handle {
     int win_cap = 0;                         // one-launch window attention workgroups resident at once
     void *scratch = nullptr;
     int built = 0;                           // tables and scratch allocated (reusable as a shell)
-    // batched prefill buffers ([TB][...] per token), allocated on first use
-    struct Batch {
-        void *buf = nullptr;
-        int TB = 0, mcb = 0;                 // tokens per attention batch, chunk capacity per q-head
-        float *x0, *x1, *q, *k, *v, *qr, *ao, *ap, *hh, *dn, *rope, *part, *part_ml;
-        int8_t *planes; int *sh, *counter, *zs;
-        int64_t *vacc, *vacc_s;
-        int64_t *gpart; int *gcnt;           // GEMM split-K partial slices and tile arrival counters
-        // batched decode over sessions (allocated on first use): logits rows,
-        // greedy tokens, per-token token / position / per-layer page tables
-        void *dbuf = nullptr;
-        float *logits; int *next, *toks, *tpos; float *const **tpages;
-        int2 *work; int nwork = 0, wcap = 0;   // full-context layers' (token, chunk) work items
-        void *hstage = nullptr;              // pinned upload staging for toks/tpos/tpages
-    } b;
+    Batch b;                                 // leased for the duration of a batched call (BatchLease)
     // graph cache: key (logits?, argmax?, grid_global, grid_local, chunk_global)
     struct GKey { int lg, am, gg, gl, cg, rt; bool operator<(const GKey &o) const {
         return std::tie(lg, am, gg, gl, cg, rt) < std::tie(o.lg, o.am, o.gg, o.gl, o.cg, o.rt); } };
@@ -802,19 +826,12 @@ int alloc_scratch(sp_kvdecode_handle *h) {
     return 0;
 }
 
-// Drop the batch buffers and captured graphs when the arithmetic mode changes
-// (both are mode-specific); everything else of the handle is mode-independent.
+// Drop the captured graphs when the arithmetic mode changes (they are
+// mode-specific); everything else of the handle is mode-independent.
 void set_handle_mode(sp_kvdecode_handle *h, int mode) {
     if (h->mode == mode) return;
     h->mode = mode;
     free_graphs(h);
-    if (h->b.buf || h->b.dbuf) {
-        hipStreamSynchronize(h->stream);
-        if (h->b.buf) hipFree(h->b.buf);
-        if (h->b.dbuf) hipFree(h->b.dbuf);
-        if (h->b.hstage) hipHostFree(h->b.hstage);
-        h->b = sp_kvdecode_handle::Batch{};
-    }
 }
 
 // A fresh pool when the stored row format changes (mode or codec, only before
@@ -933,9 +950,6 @@ void free_handle(sp_kvdecode_handle *h) {
     if (h->d_pt) hipFree(h->d_pt);
     if (h->h_pt) hipHostFree(h->h_pt);
     if (h->scratch) hipFree(h->scratch);
-    if (h->b.buf) hipFree(h->b.buf);
-    if (h->b.dbuf) hipFree(h->b.dbuf);
-    if (h->b.hstage) hipHostFree(h->b.hstage);
     if (h->h_st) hipHostFree(h->h_st);
     if (h->h_logits) hipHostFree(h->h_logits);
     if (h->stream) hipStreamDestroy(h->stream);
@@ -1135,6 +1149,38 @@ bool batch_supported(const sp_kvdecode_handle *h) {
     return true;
 }
 
+// A batched call's hold on a set of buffers (h->b).  done() says that the call
+// ended well; a set that a failed call leaves is freed, not kept.
+struct BatchLease {
+    sp_kvdecode_handle *h;
+    bool whole = false;
+    explicit BatchLease(sp_kvdecode_handle *hh) : h(hh) {
+        std::lock_guard<std::mutex> lk(h->m->batch_mu);
+        auto &v = h->m->batches;
+        for (size_t i = v.size(); i-- > 0;)
+            if ((v[i].mode == FLOAT || h->mode != FLOAT) && v[i].pmax >= h->pmax) { h->b = v[i]; v.erase(v.begin() + (ptrdiff_t)i); return; }
+        h->b.mode = h->mode; h->b.pmax = h->pmax;
+    }
+    BatchLease(const BatchLease &) = delete;
+    void done() { whole = true; }             // after the stream's synchronize
+    ~BatchLease() {
+        if (!whole) hipStreamSynchronize(h->stream);
+        Batch drop;
+        {
+            std::lock_guard<std::mutex> lk(h->m->batch_mu);
+            auto &v = h->m->batches;
+            drop = h->b;
+            if (whole && drop.buf) {
+                v.push_back(drop);
+                drop = Batch{};
+                if (v.size() > MAX_IDLE_BATCHES) { drop = v.front(); v.erase(v.begin()); }
+            }
+        }
+        drop.release();
+        h->b = Batch{};
+    }
+};
+
 int alloc_batch(sp_kvdecode_handle *h) {
     if (h->b.buf) return 0;
     const DevModel *m = h->m;
@@ -1180,11 +1226,9 @@ int run_batch(sp_kvdecode_handle *h, int T, int pos0, int pos_hi, bool multi, Ti
     auto tp = [&](bool fold) { return fold ? (T + 15) / 16 * 16 : (T + 31) / 32 * 32; };
     auto TM = [&](int cls, bool begin) { if (cb) cb(ctx, cls, begin); };
     TM(8, true);
-    launch_embed_batch(m->embd, h->tokbuf, pos0, T, b.x1, m->gemma ? sqrtf((float)m->E) : 0.0f, s,
-                       multi ? b.toks : nullptr);
-    launch_rope_table_batch(pos0, T, m->HD, h->mode, m->base, m->gemma ? 10000.0f : m->base,
-                            m->freq_global, m->gemma ? m->freq_local : m->freq_global, b.rope, s,
-                            multi ? b.tpos : nullptr);
+    launch_embed_rope_batch(m->embd, h->tokbuf, pos0, multi ? b.toks : nullptr, multi ? b.tpos : nullptr, T, b.x1,
+                            m->gemma ? sqrtf((float)m->E) : 0.0f, m->HD, h->mode,
+                            m->freq_global, m->gemma ? m->freq_local : m->freq_global, b.rope, s);
     TM(8, false);
     auto stage = [&](int kind, const float *x, const float *delta, const float *post_w, const float *norm_w,
                      float *x_out, int n, bool fold) {
@@ -1510,7 +1554,9 @@ int sp_hipkv_prefill(sp_kvdecode_handle *h, const int32_t *tokens, int n_tok) {
     HIPCHK(hipStreamSynchronize(h->stream), "prefill staging");
     HIPCHK(hipMemcpyAsync(h->tokbuf + h->dpos, tokens, (size_t)n_tok * 4, hipMemcpyHostToDevice, h->stream),
            "prefill tokens");
+    std::unique_ptr<BatchLease> lease;
     if (h->use_batch && batch_supported(h)) {
+        lease.reset(new BatchLease(h));
         if (alloc_batch(h)) return 1;
         // window layers on a ring: writing position q reuses the page slot of
         // the page ring_pages back, i.e. drops positions up to q - ring*PAGE + PAGE-1;
@@ -1528,8 +1574,31 @@ int sp_hipkv_prefill(sp_kvdecode_handle *h, const int32_t *tokens, int n_tok) {
         }
     }
     HIPCHK(hipStreamSynchronize(h->stream), "prefill");
+    if (lease) lease->done();
     h->dpos += n_tok;
     h->hwm = std::max(h->hwm, h->dpos);
+    return 0;
+}
+
+// `bytes` of the batch's logits rows to the caller's memory through the pinned
+// slots, each piece copied out while the next ones are on the bus.  Handed to the
+// runtime as one copy to pageable memory, a piece's bus transfer and its copy out
+// took turns: 64 rows of 16 384 floats 300 us, so 170.
+static int logits_to_host(sp_kvdecode_handle *h, float *dst, size_t bytes) {
+    auto &b = h->b;
+    const size_t n = (bytes + LOGIT_SLOT_BYTES - 1) / LOGIT_SLOT_BYTES;
+    auto size = [&](size_t c) { return std::min(LOGIT_SLOT_BYTES, bytes - c * LOGIT_SLOT_BYTES); };
+    for (size_t c = 0; c < n + LOGIT_SLOTS; c++) {
+        if (c >= LOGIT_SLOTS) {
+            const size_t d = c - LOGIT_SLOTS;
+            HIPCHK(hipEventSynchronize(b.slot_ev[d % LOGIT_SLOTS]), "batch logits download");
+            memcpy((uint8_t *)dst + d * LOGIT_SLOT_BYTES, b.hslots + d % LOGIT_SLOTS * LOGIT_SLOT_BYTES, size(d));
+        }
+        if (c >= n) continue;
+        HIPCHK(hipMemcpyAsync(b.hslots + c % LOGIT_SLOTS * LOGIT_SLOT_BYTES, (const uint8_t *)b.logits + c * LOGIT_SLOT_BYTES,
+                              size(c), hipMemcpyDeviceToHost, h->stream), "batch logits download");
+        HIPCHK(hipEventRecord(b.slot_ev[c % LOGIT_SLOTS], h->stream), "batch logits download");
+    }
     return 0;
 }
 
@@ -1572,22 +1641,29 @@ static int decode_batch_impl(sp_kvdecode_handle *const *hs, int n, const int32_t
         return 0;
     }
     for (int i = 0; i < n; i++) if (ensure_pages(hs[i], hs[i]->dpos, hs[i]->dpos + 1)) return 1;
+    BatchLease lease(L);
     if (alloc_batch(L)) return 1;
     auto &b = L->b;
     const int TB = b.TB;
     if (!b.dbuf) {
         const size_t lb = (size_t)TB * m->V * 4, nb = (size_t)TB * 4, pb = (size_t)m->NL * TB * sizeof(void *);
         b.wcap = TB * (L->pmax / ATTN_MAXCH + 2);
-        const size_t wb = (size_t)b.wcap * sizeof(int2);
-        HIPCHK(hipMalloc(&b.dbuf, align_up(lb, 256) + 3 * align_up(nb, 256) + align_up(pb, 256) + wb), "batch decode alloc");
+        const size_t wb = (size_t)b.wcap * sizeof(int2), up = 2 * nb + pb + wb;
+        // pinned staging: the upload block, the tokens, the logits' slots
+        // (allocated before dbuf, which marks both as present)
+        if (!b.hstage) HIPCHK(hipHostMalloc(&b.hstage, align_up(up, 4096) + align_up(nb, 4096) + LOGIT_SLOTS * LOGIT_SLOT_BYTES,
+                                            hipHostMallocDefault), "batch decode staging");
+        b.hnext = (int *)((uint8_t *)b.hstage + align_up(up, 4096));
+        b.hslots = (uint8_t *)b.hnext + align_up(nb, 4096);
+        for (hipEvent_t &e : b.slot_ev) if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming), "batch decode event");
+        HIPCHK(hipMalloc(&b.dbuf, align_up(lb, 256) + align_up(nb, 256) + up), "batch decode alloc");
         uint8_t *p = (uint8_t *)b.dbuf;
         b.logits = (float *)p; p += align_up(lb, 256);
         b.next = (int *)p; p += align_up(nb, 256);
-        b.toks = (int *)p; p += align_up(nb, 256);
-        b.tpos = (int *)p; p += align_up(nb, 256);
-        b.tpages = (float *const **)p; p += align_up(pb, 256);
+        b.toks = (int *)p; p += nb;
+        b.tpos = (int *)p; p += nb;
+        b.tpages = (float *const **)p; p += pb;
         b.work = (int2 *)p;
-        HIPCHK(hipHostMalloc(&b.hstage, 2 * nb + pb + wb, hipHostMallocDefault), "batch decode staging");
     }
     for (int g0 = 0; g0 < n; g0 += TB) {
         const int T = std::min(TB, n - g0);
@@ -1604,24 +1680,22 @@ static int decode_batch_impl(sp_kvdecode_handle *const *hs, int n, const int32_t
             // full-context layers: ATTN_MAXCH-position chunks up to this session's position
             for (int c = 0; c <= h->dpos / ATTN_MAXCH && b.nwork < b.wcap; c++) hwork[b.nwork++] = make_int2(t, c);
         }
-        HIPCHK(hipMemcpyAsync(b.toks, htok, (size_t)TB * 4, hipMemcpyHostToDevice, L->stream), "batch tokens");
-        HIPCHK(hipMemcpyAsync(b.tpos, hpos, (size_t)TB * 4, hipMemcpyHostToDevice, L->stream), "batch positions");
-        HIPCHK(hipMemcpyAsync((void *)b.tpages, hpg, (size_t)m->NL * TB * sizeof(void *), hipMemcpyHostToDevice, L->stream),
-               "batch page tables");
-        HIPCHK(hipMemcpyAsync(b.work, hwork, (size_t)b.nwork * sizeof(int2), hipMemcpyHostToDevice, L->stream),
-               "batch work items");
+        // tokens, positions, page tables and work items lie in one block on both sides
+        HIPCHK(hipMemcpyAsync(b.toks, htok, (size_t)((uint8_t *)(hwork + b.nwork) - (uint8_t *)htok), hipMemcpyHostToDevice,
+                              L->stream), "batch upload");
         if (run_batch(L, T, 0, pos_hi, true, cb, ctx)) return 1;
-        if (logits) HIPCHK(hipMemcpyAsync(logits + (size_t)g0 * m->V, b.logits, (size_t)T * m->V * 4,
-                                          hipMemcpyDeviceToHost, L->stream), "batch logits download");
-        if (next_tokens) HIPCHK(hipMemcpyAsync(next_tokens + g0, b.next, (size_t)T * 4, hipMemcpyDeviceToHost, L->stream),
+        if (next_tokens) HIPCHK(hipMemcpyAsync(b.hnext, b.next, (size_t)T * 4, hipMemcpyDeviceToHost, L->stream),
                                 "batch tokens download");
+        if (logits && logits_to_host(L, logits + (size_t)g0 * m->V, (size_t)T * m->V * 4)) return 1;
         HIPCHK(hipStreamSynchronize(L->stream), "batch decode");
+        if (next_tokens) memcpy(next_tokens + g0, b.hnext, (size_t)T * 4);
         for (int t = 0; t < T; t++) {
             sp_kvdecode_handle *h = hs[g0 + t];
             h->dpos++;
             h->hwm = std::max(h->hwm, h->dpos);
         }
     }
+    lease.done();
     return 0;
 }
 

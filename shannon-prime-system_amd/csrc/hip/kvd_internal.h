@@ -271,13 +271,8 @@ void launch_fail(const char *msg);
 const char *launch_take_error();
 
 // launchers (kvd_kernels.hip)
-void launch_embed(const DevW &embd, const DState *st, const int *tokbuf, float *x, float scale, hipStream_t s,
-                  VecStat *stats = nullptr, int nstats = 0);
-void launch_embed_batch(const DevW &embd, const int *tokbuf, int pos0, int T, float *x, float scale, hipStream_t s,
-                        const int *toks = nullptr);
-void launch_rope_table_batch(int pos0, int T, int HD, int mode, float base_g, float base_l,
-                             const int64_t *fq_g, const int64_t *fq_l, float *out, hipStream_t s,
-                             const int *tpos = nullptr);
+void launch_embed_rope_batch(const DevW &embd, const int *tokbuf, int pos0, const int *toks, const int *tpos, int T, float *x,
+                             float scale, int HD, int mode, const int64_t *fq_g, const int64_t *fq_l, float *rope, hipStream_t s);
 void launch_argmax_rows(const float *logits, int V, int T, int *out, hipStream_t s);
 void launch_stage(const StageArgs &a, hipStream_t s);
 void launch_gemm(const GemmArgs &a, int nrows_total, hipStream_t s);
@@ -294,8 +289,6 @@ void attn_time_next(hipEvent_t start, hipEvent_t stop);   // ... and of its next
 void launch_qk_prep(const AttnArgs &a, hipStream_t s);
 void launch_embed_rope(const DevW &embd, const DState *st, const int *tokbuf, float *x, float scale, VecStat *stats,
                        int nstats, int HD, int mode, const int64_t *fq_g, const int64_t *fq_l, float *rope, hipStream_t s);
-void launch_rope_table(const DState *st, int HD, int mode, float base_g, float base_l,
-                       const int64_t *fq_g, const int64_t *fq_l, float *out, hipStream_t s);
 void launch_attention(const AttnArgs &a, int grid_chunks, hipStream_t s);
 int  attn_capacity(int HD, int G);
 int  window_capacity(int HD, int G);   // workgroups of the one-launch window attention resident at once (0: none)
