@@ -64,15 +64,18 @@ __device__ __forceinline__ void digits4(int32_t x, int32_t d[4]) {
 }
 
 // ---------------------------------------------------------------- score pass
-// grid: (token groups of 64 / G tokens, 64-position chunks, kv heads); the
-// token group runs fastest, so the groups reading one chunk's K run together.
+// grid: (kv heads, token groups of 64 / G tokens, 64-position chunks).  The head
+// runs fastest: workgroups go to the 8 XCDs in turn, so with 8 kv heads each
+// XCD's L2 serves one head's rows (all heads' together are more than it holds:
+// 9 MB of V for a window pass at the Gemma-3-12B shape against 4 MB); then the
+// token group, so the groups reading one chunk's K run together.
 // zscratch and the chunk maxima are laid out per token as for the decode
 // kernels: token t's scores at zscratch + t NH zstride, its maximum of chunk c
 // of token-head q at part_ml + t NH max_chunks 4 + (q max_chunks + c) 4.
 template <int EPL, int G>
 __global__ __launch_bounds__(256) void k_pattn_scores(AttnArgs a) {
     constexpr int HD = EPL * 64, KS = HD / 32, TPW = 16 / G, TWG = 4 * TPW, KROW = HD + 16;
-    const int tg = blockIdx.x, c = win_start(a, 0) / PS_CH + (int)blockIdx.y, h = blockIdx.z;
+    const int h = blockIdx.x, tg = blockIdx.y, c = win_start(a, 0) / PS_CH + (int)blockIdx.z;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t0 = tg * TWG;
     const int tend = t0 + TWG < a.nt ? t0 + TWG : a.nt;
@@ -241,7 +244,7 @@ __global__ __launch_bounds__(256) void k_pattn_scores(AttnArgs a) {
 }
 
 // --------------------------------------------------------------- V-sum pass
-// grid: (token groups of TT tokens, 2048-position chunks, kv heads).  NQ =
+// grid: (kv heads, token groups of TT tokens, 2048-position chunks).  NQ =
 // TT G token-heads share each V row.  Token t's totals are its decode-layout
 // accumulators (vacc + t QD VREP, vacc_s + t NH VREP, replica 0) and its
 // group's arrivals count on counter[t0 NKV + h].
@@ -252,7 +255,7 @@ template <int EPL, int G, int TT, bool WIN>
 __global__ __launch_bounds__(WIN ? 512 : 256) void k_pattn_vsum(AttnArgs a) {
     constexpr int HD = EPL * 64, NQ = TT * G, UV = WIN ? 8 : 4, NW = WIN ? 8 : 4, NT = 64 * NW;
     const int VC = PV_CH;
-    const int tg = blockIdx.x, c = win_start(a, 0) / VC + (int)blockIdx.y, h = blockIdx.z;
+    const int h = blockIdx.x, tg = blockIdx.y, c = win_start(a, 0) / VC + (int)blockIdx.z;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t0 = tg * TT;
     const int tend = t0 + TT < a.nt ? t0 + TT : a.nt;
@@ -264,14 +267,17 @@ __global__ __launch_bounds__(WIN ? 512 : 256) void k_pattn_vsum(AttnArgs a) {
     const int cs = WIN ? s0g : (c * VC > s0g ? c * VC : s0g);
     const int np = WIN ? pos_hi - s0g + 1 : (pos_hi < c * VC + VC - 1 ? pos_hi : c * VC + VC - 1) - cs + 1;
     const size_t QD = (size_t)a.NH * HD;
-    __shared__ int32_t ew[NQ][PV_SUB + UV];              // island weights (Q22) of a sub-chunk, 0 where masked and past it
+    // island weights (Q22) of a sub-chunk, 0 where masked and past it: a row's
+    // NQ side by side (a wave reads them with NQ / 2 16-byte loads) and as
+    // doubles, converted once (every wave converted each again per row)
+    __shared__ __align__(16) double ew[PV_SUB + UV][NQ];
     __shared__ int s_M[NQ];
     __shared__ int64_t ored[NQ][HD];                      // the waves' partials, added in LDS (order-free)
     __shared__ int64_t sred[NQ];
     __shared__ int is_last;
     for (int i = threadIdx.x; i < NQ * HD; i += NT) ored[i / HD][i % HD] = 0;
     if (threadIdx.x < NQ) sred[threadIdx.x] = 0;
-    if (threadIdx.x < NQ * UV) ew[threadIdx.x / UV][PV_SUB + threadIdx.x % UV] = 0;
+    if (threadIdx.x < NQ * UV) ew[PV_SUB + threadIdx.x / NQ][threadIdx.x % NQ] = 0.0;
     // each token-head's maximum over its 64-position chunk maxima (wave w: token-heads w, w+4, ..)
     for (int q = wave; q < NQ; q += NW) {
         const int tt = t0 + q / G;
@@ -291,23 +297,31 @@ __global__ __launch_bounds__(WIN ? 512 : 256) void k_pattn_vsum(AttnArgs a) {
         // the sub-chunk's scores: every slot's load is issued first (token and
         // position clamped into range, masked slots' values unused), then the
         // weights are formed -- one round trip, not one per slot
-        static_assert(NQ * PV_SUB % NT == 0, "whole slots per thread");
-        constexpr int FPT = NQ * PV_SUB / NT;
-        int32_t zz[FPT];
+        // thread i takes rows i, i + NT of every token-head (coalesced along the row)
+        static_assert(PV_SUB % NT == 0, "whole rows per thread");
+        constexpr int RPT = PV_SUB / NT;
+        int32_t zz[NQ * RPT];
         #pragma unroll
-        for (int k = 0; k < FPT; k++) {
-            const int i = threadIdx.x + NT * k, q = i / PV_SUB, jj = i % PV_SUB;
+        for (int k = 0; k < NQ * RPT; k++) {
+            const int q = k / RPT, jj = threadIdx.x + NT * (k % RPT);
             const int tt = t0 + q / G < a.nt ? t0 + q / G : a.nt - 1;
             const int p = cs + sb + (jj < ns ? jj : ns - 1);
             zz[k] = a.zscratch[(size_t)tt * a.NH * a.zstride + (size_t)(h * G + q % G) * a.zstride + p];
         }
         #pragma unroll
-        for (int k = 0; k < FPT; k++) {
-            const int i = threadIdx.x + NT * k, q = i / PV_SUB, jj = i % PV_SUB, tt = t0 + q / G, p = cs + sb + jj;
-            int32_t w = 0;
-            if (jj < ns && tt < a.nt && p <= a.pos0 + tt && p >= win_start(a, tt))
-                w = (int32_t)(exp_fixed((((int64_t)zz[k] - (int64_t)s_M[q]) * ONE) >> 14) >> 8);
-            ew[q][jj] = w;
+        for (int q = 0; q < NQ; q++) {
+            int64_t sum = 0;
+            #pragma unroll
+            for (int r = 0; r < RPT; r++) {
+                const int jj = threadIdx.x + NT * r, tt = t0 + q / G, p = cs + sb + jj;
+                int32_t w = 0;
+                if (jj < ns && tt < a.nt && p <= a.pos0 + tt && p >= win_start(a, tt))
+                    w = (int32_t)(exp_fixed((((int64_t)zz[q * RPT + r] - (int64_t)s_M[q]) * ONE) >> 14) >> 8);
+                ew[jj][q] = (double)w;
+                sum += w;
+            }
+            sum = wave_allsum(sum);                      // the sub-chunk's denominators
+            if (lane == 0) atomicAdd((unsigned long long *)&sred[q], (unsigned long long)sum);
         }
         __syncthreads();
         // FP64 V-sum of the sub-chunk: a wave's rows (<= 128) keep every
@@ -347,7 +361,7 @@ __global__ __launch_bounds__(WIN ? 512 : 256) void k_pattn_vsum(AttnArgs a) {
             for (int u = 0; u < UV; u++) {
                 #pragma unroll
                 for (int q = 0; q < NQ; q++) {
-                    const double w = (double)ew[q][j0 + u];
+                    const double w = ew[j0 + u][q];
                     #pragma unroll
                     for (int e = 0; e < EPL; e++) o[q][e] = fma(w, (double)v[u][e], o[q][e]);
                 }
@@ -370,13 +384,6 @@ __global__ __launch_bounds__(WIN ? 512 : 256) void k_pattn_vsum(AttnArgs a) {
         for (int q = 0; q < NQ; q++)
             #pragma unroll
             for (int e = 0; e < EPL; e++) atomicAdd((unsigned long long *)&ored[q][lane * EPL + e], (unsigned long long)(int64_t)o[q][e]);
-        // denominators of the sub-chunk
-        for (int q = wave; q < NQ; q += NW) {
-            int64_t sum = 0;
-            for (int jj = lane; jj < PV_SUB; jj += 64) sum += ew[q][jj];
-            sum = wave_allsum(sum);
-            if (lane == 0) atomicAdd((unsigned long long *)&sred[q], (unsigned long long)sum);
-        }
         __syncthreads();                                 // ew is consumed
     }
     if constexpr (WIN) {
@@ -427,12 +434,12 @@ template <int EPL, int G>
 void pattn_go(const AttnArgs &a, hipStream_t s) {
     constexpr int TPW = 16 / G, TWG = 4 * TPW, TT = 8 / G;
     const int pos_hi = a.pos0 + a.nt - 1, lo = win_start(a, 0);
-    const dim3 g1((a.nt + TWG - 1) / TWG, pos_hi / PS_CH - lo / PS_CH + 1, a.NKV);
+    const dim3 g1(a.NKV, (a.nt + TWG - 1) / TWG, pos_hi / PS_CH - lo / PS_CH + 1);
     hipLaunchKernelGGL((k_pattn_scores<EPL, G>), g1, dim3(256), 0, s, a);
     if (a.win >= 0) {
-        hipLaunchKernelGGL((k_pattn_vsum<EPL, G, TT, true>), dim3((a.nt + TT - 1) / TT, 1, a.NKV), dim3(512), 0, s, a);
+        hipLaunchKernelGGL((k_pattn_vsum<EPL, G, TT, true>), dim3(a.NKV, (a.nt + TT - 1) / TT), dim3(512), 0, s, a);
     } else {
-        const dim3 g2((a.nt + TT - 1) / TT, pos_hi / PV_CH - lo / PV_CH + 1, a.NKV);
+        const dim3 g2(a.NKV, (a.nt + TT - 1) / TT, pos_hi / PV_CH - lo / PV_CH + 1);
         hipLaunchKernelGGL((k_pattn_vsum<EPL, G, TT, false>), g2, dim3(256), 0, s, a);
     }
 }

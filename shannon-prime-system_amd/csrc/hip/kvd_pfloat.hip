@@ -62,18 +62,19 @@ __device__ __forceinline__ bool finite4(const v4f &v) {
 
 }  // namespace
 
-// grid: (token tiles, position splits, kv heads)
+// grid: (kv heads, token tiles, position splits); with 8 kv heads each XCD
+// (workgroups go to the 8 of them in turn) reads one head's rows
 template <int EPL, int G>
 __global__ __launch_bounds__(64 * PF_WAVES, 2) void k_pfloat(AttnArgs a, int nsplit) {
     constexpr int HD = EPL * 64, CPR = HD / 16, TOK = PF_ROWS / G;     // CPR: 16-float groups of a row
     constexpr int PIECES = PF_POS * HD / 4;                            // 16-byte pieces of a K or V tile
     __shared__ __align__(1024) v4f kv[2][2][PIECES];                   // [buffer][K, V][position][piece ^ position % 16]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l16 = lane & 15, g = lane >> 4, h = blockIdx.z;
-    const int t0 = (int)blockIdx.x * TOK, tend = t0 + TOK < a.nt ? t0 + TOK : a.nt;
+    const int l16 = lane & 15, g = lane >> 4, h = blockIdx.x;
+    const int t0 = (int)blockIdx.y * TOK, tend = t0 + TOK < a.nt ? t0 + TOK : a.nt;
     // this split's tiles of the token tile's span [start, last]
     const int last = a.pos0 + tend - 1, lo = start_of(a, t0) / PF_POS, hi = last / PF_POS + 1;
-    const int per = (hi - lo + nsplit - 1) / nsplit, b0 = lo + (int)blockIdx.y * per, b1 = b0 + per < hi ? b0 + per : hi;
+    const int per = (hi - lo + nsplit - 1) / nsplit, b0 = lo + (int)blockIdx.z * per, b1 = b0 + per < hi ? b0 + per : hi;
     // this lane's token-head, and the wave's token range
     const int row = wave * 16 + l16, tq = t0 + row / G, head = h * G + row % G;
     const bool live = tq < tend;
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void k_pfloat(AttnArgs a, int nsp
         const int r = wave * 16 + 4 * g + i, t = t0 + r / G, hd = h * G + r % G;
         const float lr = __shfl(l, 4 * g + i, 64), mr = __shfl(m, 4 * g + i, 64);
         if (t >= tend) continue;
-        const size_t at = ((size_t)t * a.NH + hd) * nsplit + blockIdx.y;
+        const size_t at = ((size_t)t * a.NH + hd) * nsplit + blockIdx.z;
         float *out = nsplit > 1 ? a.part + at * HD : a.ao + (size_t)t * QD + (size_t)hd * HD;
         #pragma unroll
         for (int u = 0; u < HD / 64; u++) {
@@ -263,7 +264,7 @@ static void pfloat_go(const AttnArgs &a, hipStream_t s) {
     const int room = (int)std::min<size_t>((size_t)a.part_tokens * a.max_chunks / a.nt, 64);
     int n = (512 + tiles * a.NKV - 1) / (tiles * a.NKV);
     n = std::max(1, std::min(std::min(n, span / 2), room));
-    const dim3 grid(tiles, n, a.NKV), wg(64 * PF_WAVES);
+    const dim3 grid(a.NKV, tiles, n), wg(64 * PF_WAVES);
     hipLaunchKernelGGL((k_pfloat<EPL, G>), grid, wg, 0, s, a, n);
     if (n > 1) hipLaunchKernelGGL(k_pfloat_merge, dim3(a.nt * a.NH), dim3(a.HD), 0, s, a, n);
 }
