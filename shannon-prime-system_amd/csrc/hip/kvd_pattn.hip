@@ -9,10 +9,16 @@
 //   w = exp_fixed(((z - M) 2^30) >> 14) >> 8 (Q22), M the token-head's max;
 //   out = RNE(sum_p w vq / (sum_p w * 2^16)).
 //
-// Score pass, on the int8 matrix cores: qi and ki are split into four balanced
-// base-256 digits; every digit pair (a, b) is one int8 MFMA product with an
-// exact int32 sum (|sum| <= HD 2^14), and ip = sum_{a,b} 2^(8(a+b)) P_ab in
-// int64 -- the same integer as the decode kernels' int64 dot product.  A
+// Score pass, on the int8 matrix cores: qi and ki are split into balanced
+// base-256 digits, three where every value of the workgroup fits (|x| <= 127 (1 +
+// 2^8 + 2^16): |q|, |k| below 127) and four otherwise; every digit pair (a, b) is
+// one int8 MFMA product with an exact int32 sum (|sum| <= HD 2^14), and ip =
+// sum_{a,b} 2^(8(a+b)) P_ab in int64 -- the same integer as the decode kernels'
+// int64 dot product.  Forming the digits bounds the pass (each q row's once per
+// 64 positions, each K row's once per 64 token-heads), then the products: three
+// digits need 9 of them, four 16.  128 tokens of Gemma-3-12B's window layers at
+// position 1024 and up, 18 chunks x 8 kv heads: 32.8 -> 26.4 us against four
+// digits always, formed by a shift and a subtraction each.  A
 // workgroup scores 64 positions for 64 token-heads (one 16 x 16 tile row per
 // wave); the positions' K digits are staged once in LDS.  A workgroup whose q
 // or K values do not fit four balanced digits (|x| > 127 (1 + 2^8 + 2^16 +
@@ -32,6 +38,7 @@
 #include "kvd_exact.h"
 #include "kvd_vec.h"
 #include "kvd_spinor.h"
+#include <type_traits>
 
 namespace kvd {
 
@@ -43,6 +50,7 @@ constexpr int PS_CH = 64;            // positions per score workgroup (and per c
 constexpr int PV_CH = 2048;          // positions per V-sum workgroup (full-context layers)
 constexpr int PV_SUB = 512;          // ... in sub-chunks of 128 rows per wave (FP64 sums below 2^53)
 constexpr int DIG_MAX = 127 * (1 + 256 + 65536 + 16777216);   // largest |x| of four balanced digits
+constexpr int DIG3_MAX = 127 * (1 + 256 + 65536);             // ... of three
 
 __device__ __forceinline__ const float *pg(const AttnArgs &a, int pos) {
     const int lp = pos / PAGE;
@@ -54,13 +62,20 @@ __host__ __device__ __forceinline__ int win_start(const AttnArgs &a, int t) {
     return a.win >= 0 && q > 0 ? q : 0;
 }
 
-// x = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3, d in [-128, 127] (|x| <= DIG_MAX)
-__device__ __forceinline__ void digits4(int32_t x, int32_t d[4]) {
-    #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        d[k] = ((x + 128) & 255) - 128;
-        x = (x - d[k]) >> 8;
-    }
+// x = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3, d in [-128, 127] (|x| <= DIG_MAX), the
+// digits as bytes: adding 128 to each byte place with carries gives d + 128
+__device__ __forceinline__ uint32_t digits4(int32_t x) { return ((uint32_t)x + 0x80808080u) ^ 0x80808080u; }
+// four values' digits -> one dword per digit place (byte e = value e)
+__device__ __forceinline__ void digit_planes(const int32_t x[4], uint32_t w[4]) {
+    const uint32_t a = digits4(x[0]), b = digits4(x[1]), c = digits4(x[2]), d = digits4(x[3]);
+    const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u), ab2 = __builtin_amdgcn_perm(b, a, 0x07030602u);
+    const uint32_t cd0 = __builtin_amdgcn_perm(d, c, 0x05010400u), cd2 = __builtin_amdgcn_perm(d, c, 0x07030602u);
+    w[0] = __builtin_amdgcn_perm(cd0, ab0, 0x05040100u); w[1] = __builtin_amdgcn_perm(cd0, ab0, 0x07060302u);
+    w[2] = __builtin_amdgcn_perm(cd2, ab2, 0x05040100u); w[3] = __builtin_amdgcn_perm(cd2, ab2, 0x07060302u);
+}
+// whether |x| needs a fourth digit (1) or more than four (2)
+__device__ __forceinline__ int digit_level(int32_t x) {
+    return ((uint32_t)x + (uint32_t)DIG3_MAX > 2u * DIG3_MAX ? 1 : 0) | ((uint32_t)x + (uint32_t)DIG_MAX > 2u * DIG_MAX ? 2 : 0);
 }
 
 // ---------------------------------------------------------------- score pass
@@ -74,7 +89,7 @@ __device__ __forceinline__ void digits4(int32_t x, int32_t d[4]) {
 // of token-head q at part_ml + t NH max_chunks 4 + (q max_chunks + c) 4.
 template <int EPL, int G>
 __global__ __launch_bounds__(256) void k_pattn_scores(AttnArgs a) {
-    constexpr int HD = EPL * 64, KS = HD / 32, TPW = 16 / G, TWG = 4 * TPW, KROW = HD + 16;
+    constexpr int HD = EPL * 64, KS = HD / 64, TPW = 16 / G, TWG = 4 * TPW, KROW = HD + 16;
     const int h = blockIdx.x, tg = blockIdx.y, c = win_start(a, 0) / PS_CH + (int)blockIdx.z;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t0 = tg * TWG;
@@ -84,26 +99,31 @@ __global__ __launch_bounds__(256) void k_pattn_scores(AttnArgs a) {
     if (t0 >= a.nt || cs > pos_hi || cs + PS_CH <= win_start(a, t0)) return;
     const int np = pos_hi - cs + 1 < PS_CH ? pos_hi - cs + 1 : PS_CH;
     __shared__ __align__(16) int8_t kd[4][PS_CH][KROW];   // K digits [digit][position][dim]
-    __shared__ int s_wide;
-    if (threadIdx.x == 0) s_wide = 0;
+    __shared__ int s_level;
+    if (threadIdx.x == 0) s_level = 0;
     const size_t QD = (size_t)a.NH * HD;
     // this wave's 16 token-heads: lane row m = lane % 16 -> token t0 + wave TPW + m / G, head h G + m % G
     const int m = lane & 15, j = lane >> 4;
     const int tq = t0 + wave * TPW + m / G;
-    const float *qp = a.qr + (size_t)(tq < a.nt ? tq : 0) * QD + (size_t)(h * G + m % G) * HD + 8 * j;
-    int32_t qi[KS][8];
-    bool wide = false;
+    // its A operands: digit b of qi at dims 64 ks + 16 j .. + 16
+    const float *qp = a.qr + (size_t)(tq < a.nt ? tq : 0) * QD + (size_t)(h * G + m % G) * HD + 16 * j;
+    v4i A[4][KS];
+    int level = 0;
     #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        const float4 v0 = *(const float4 *)(qp + 32 * ks), v1 = *(const float4 *)(qp + 32 * ks + 4);
-        const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+    for (int ks = 0; ks < KS; ks++)
         #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            qi[ks][e] = tq < a.nt ? (int32_t)rintf(v[e] * 65536.0f) : 0;
-            wide |= qi[ks][e] > DIG_MAX || qi[ks][e] < -DIG_MAX;
+        for (int q = 0; q < 4; q++) {
+            const float4 v = *(const float4 *)(qp + 64 * ks + 4 * q);
+            int32_t x[4] = {(int32_t)rintf(v.x * 65536.0f), (int32_t)rintf(v.y * 65536.0f),
+                            (int32_t)rintf(v.z * 65536.0f), (int32_t)rintf(v.w * 65536.0f)};
+            uint32_t w[4];
+            #pragma unroll
+            for (int e = 0; e < 4; e++) { if (tq >= a.nt) x[e] = 0; level |= digit_level(x[e]); }
+            digit_planes(x, w);
+            #pragma unroll
+            for (int b = 0; b < 4; b++) A[b][ks][q] = (int)w[b];
         }
-    }
-    __syncthreads();                                    // s_wide is cleared
+    __syncthreads();                                    // s_level is cleared
     // K rows of the chunk as digit planes: thread i takes 16 consecutive dims of
     // a row.  The chunk is one page (PS_CH == PAGE, chunks aligned), looked up
     // once; every row load is requested before the first is used, rows past
@@ -129,73 +149,58 @@ __global__ __launch_bounds__(256) void k_pattn_scores(AttnArgs a) {
     #pragma unroll
     for (int it = 0; it < KIT; it++) {
         const int i = threadIdx.x + 256 * it, pl = i / (HD / 16), d0 = (i % (HD / 16)) * 16;
-        int32_t x[16];
+        uint32_t w[4][4];
         #pragma unroll
         for (int q = 0; q < 4; q++) {
-            x[4 * q] = kx[it][q].x ^ after_loads; x[4 * q + 1] = kx[it][q].y ^ after_loads;
-            x[4 * q + 2] = kx[it][q].z ^ after_loads; x[4 * q + 3] = kx[it][q].w ^ after_loads;
-        }
-        uint32_t w[4][4] = {};
-        #pragma unroll
-        for (int e = 0; e < 16; e++) {
-            wide |= x[e] > DIG_MAX || x[e] < -DIG_MAX;
-            int32_t d[4];
-            digits4(x[e], d);
+            const int32_t x[4] = {kx[it][q].x ^ after_loads, kx[it][q].y ^ after_loads, kx[it][q].z ^ after_loads, kx[it][q].w ^ after_loads};
+            uint32_t d[4];
             #pragma unroll
-            for (int b = 0; b < 4; b++) w[b][e >> 2] |= (uint32_t)(d[b] & 255) << (8 * (e & 3));
+            for (int e = 0; e < 4; e++) level |= digit_level(x[e]);
+            digit_planes(x, d);
+            #pragma unroll
+            for (int b = 0; b < 4; b++) w[b][q] = d[b];
         }
         #pragma unroll
         for (int b = 0; b < 4; b++) *(uint4 *)&kd[b][pl][d0] = make_uint4(w[b][0], w[b][1], w[b][2], w[b][3]);
     }
-    if (__any(wide) && lane == 0) s_wide = 1;
+    if (__any(level & 1) && lane == 0) atomicOr(&s_level, 1);
+    if (__any(level & 2) && lane == 0) atomicOr(&s_level, 2);
     __syncthreads();
-    const bool mfma = s_wide == 0;
-
-    // this wave's A operands: digit a of qi at dims 32 ks + 8 j .. +8 (byte e = dim 8 j + e)
-    long A[4][KS];
-    #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        uint32_t lo[4] = {}, hi[4] = {};
+    const int lvl = __builtin_amdgcn_readfirstlane(s_level);
+    // the digit products of tile nt: ND digits of q by ND of K
+    auto dots = [&](auto nd, int nt, int64_t (&ip)[4]) {
+        constexpr int ND = decltype(nd)::value;
+        v4i acc[ND * ND];
         #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            int32_t d[4];
-            digits4(qi[ks][e], d);
+        for (int k = 0; k < ND * ND; k++) acc[k] = (v4i){0, 0, 0, 0};
+        #pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            v4i B[ND];
             #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const uint32_t byte = (uint32_t)(d[b] & 255) << (8 * (e & 3));
-                if (e < 4) lo[b] |= byte; else hi[b] |= byte;
-            }
+            for (int b = 0; b < ND; b++) B[b] = *(const v4i *)&kd[b][nt * 16 + m][64 * ks + 16 * j];
+            #pragma unroll
+            for (int a2 = 0; a2 < ND; a2++)
+                #pragma unroll
+                for (int b = 0; b < ND; b++)
+                    acc[a2 * ND + b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[a2][ks], B[b], acc[a2 * ND + b], 0, 0, 0);
         }
         #pragma unroll
-        for (int b = 0; b < 4; b++) A[b][ks] = (long)(((uint64_t)hi[b] << 32) | lo[b]);
-    }
+        for (int i = 0; i < 4; i++)
+            #pragma unroll
+            for (int a2 = 0; a2 < ND; a2++)
+                #pragma unroll
+                for (int b = 0; b < ND; b++) ip[i] += (int64_t)acc[a2 * ND + b][i] * ((int64_t)1 << (8 * (a2 + b)));
+    };
     int mx[4] = {INT32_MIN, INT32_MIN, INT32_MIN, INT32_MIN};
     const int rowq = 4 * j;                              // output rows 4 j .. 4 j + 3 of the tile
     for (int nt = 0; nt < PS_CH / 16; nt++) {
         if (nt * 16 >= np) break;
         const int p = cs + nt * 16 + m;                  // this lane's output column (position)
         int64_t ip[4] = {0, 0, 0, 0};
-        if (mfma) {
-            v4i acc[16];
-            #pragma unroll
-            for (int k = 0; k < 16; k++) acc[k] = (v4i){0, 0, 0, 0};
-            #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                long B[4];
-                #pragma unroll
-                for (int b = 0; b < 4; b++) B[b] = *(const long *)&kd[b][nt * 16 + m][32 * ks + 8 * j];
-                #pragma unroll
-                for (int a2 = 0; a2 < 4; a2++)
-                    #pragma unroll
-                    for (int b = 0; b < 4; b++)
-                        acc[a2 * 4 + b] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A[a2][ks], B[b], acc[a2 * 4 + b], 0, 0, 0);
-            }
-            #pragma unroll
-            for (int i = 0; i < 4; i++)
-                #pragma unroll
-                for (int a2 = 0; a2 < 4; a2++)
-                    #pragma unroll
-                    for (int b = 0; b < 4; b++) ip[i] += (int64_t)acc[a2 * 4 + b][i] * ((int64_t)1 << (8 * (a2 + b)));
+        if (lvl == 0) {
+            dots(std::integral_constant<int, 3>{}, nt, ip);
+        } else if (lvl == 1) {
+            dots(std::integral_constant<int, 4>{}, nt, ip);
         } else {
             // out-of-range magnitudes: the tile on the vector units, from the
             // digits (x = sum_b 2^(8b) d_b exactly holds only in range, so the
