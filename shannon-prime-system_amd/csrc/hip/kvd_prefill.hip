@@ -32,11 +32,22 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 // [lane = 16 g + token % 16][16 bytes]: columns 16 m .. 16 m + 15 of block
 // 4 s + g, each 8 in the order 0 1 4 5 2 3 6 7 -- the MFMA A operand as a wave
 // reads it, 1 KiB per operand.
+// Workgroup -> token.  A token writes 8 bytes here and there of the lines its
+// tile's 16 tokens share, so where 128 tokens or more give every XCD a whole tile
+// (workgroups go to the XCDs in turn), a tile's tokens go to one XCD and its L2
+// puts the lines together.  Bound by the scattered writes: 512 tokens of 4 096 and
+// 15 360 inputs, 17.6 -> 11.2 us on average; with fewer than 128 tokens some XCDs
+// would be left without work, and the launch is bound by latency.
+__device__ __forceinline__ int stage_token(int i, int TP) {
+    if (i >= (TP & ~127)) return i;
+    const int x = i & 7, k = i >> 3;
+    return ((k >> 4) * 8 + x) * 16 + (k & 15);
+}
 template <int PRO, bool FOLD>
 __global__ __launch_bounds__(512) void k_stage(StageArgs a) {
     extern __shared__ float xf[];                      // pro.n floats (norm prologues)
     __shared__ double red[RED_SLOTS * RED_WAVES];
-    const int t = blockIdx.x, n = a.pro.n, nblk = n / 32, tid = threadIdx.x;
+    const int t = stage_token(blockIdx.x, a.TP), n = a.pro.n, nblk = n / 32, tid = threadIdx.x;
     int8_t *planes = a.planes;
     // byte offset of 8-column group g of plane pl for this token
     auto at = [&](int pl, int g) -> size_t {
