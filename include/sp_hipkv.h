@@ -187,7 +187,7 @@ int  sp_hipkv_set_graph(sp_kvdecode_handle *h, int on);
  * 32 x n_kv_heads workgroups could not be resident at once.  No counterpart in
  * the reference (a CPU attention). */
 int  sp_hipkv_set_window_one_launch(sp_kvdecode_handle *h, int on);
-/* Prefill through the batched path (1, default: 128 tokens per pass, int8-MFMA
+/* Prefill through the batched path (1, default: 512 tokens per pass, int8-MFMA
  * GEMMs, token-batched attention) or one decode step per token (0).  Both
  * leave the same K/V (bit-identical in exact mode). */
 int  sp_hipkv_set_batch_prefill(sp_kvdecode_handle *h, int on);

@@ -481,7 +481,7 @@ __global__ __launch_bounds__(256) void k_attn_float(AttnArgs a_in) {
     // (one at a time where their weights don't fit wk): wave k forms head k's
     // chunk weights, then every thread sums its outputs with 16 partials in
     // flight.  One head after the other with 4 in flight, the merge was two
-    // thirds of the kernel at 4 096 positions of the Qwen3-0.6B shape (26.2 ->
+    // thirds of the kernel at 4 096 positions of the Qwen3-0.6B shape (26 ->
     // 17 us).  The sums' order is the same.
     StatAcc sacc;
     __shared__ float sL[G];
