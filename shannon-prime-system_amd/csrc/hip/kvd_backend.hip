@@ -1647,7 +1647,7 @@ static int decode_batch_impl(sp_kvdecode_handle *const *hs, int n, const int32_t
     const int TB = b.TB;
     if (!b.dbuf) {
         const size_t lb = (size_t)TB * m->V * 4, nb = (size_t)TB * 4, pb = (size_t)m->NL * TB * sizeof(void *);
-        b.wcap = TB * (L->pmax / ATTN_MAXCH + 2);
+        b.wcap = TB * (b.pmax / ATTN_MAXCH + 2);             // the set outlives this call: its own pmax
         const size_t wb = (size_t)b.wcap * sizeof(int2), up = 2 * nb + pb + wb;
         // pinned staging: the upload block, the tokens, the logits' slots
         // (allocated before dbuf, which marks both as present)
@@ -1678,7 +1678,10 @@ static int decode_batch_impl(sp_kvdecode_handle *const *hs, int n, const int32_t
             pos_hi = std::max(pos_hi, h->dpos);
             for (int l = 0; l < m->NL; l++) hpg[(size_t)l * TB + t] = h->d_pt + h->pt_off[l];
             // full-context layers: ATTN_MAXCH-position chunks up to this session's position
-            for (int c = 0; c <= h->dpos / ATTN_MAXCH && b.nwork < b.wcap; c++) hwork[b.nwork++] = make_int2(t, c);
+            for (int c = 0; c <= h->dpos / ATTN_MAXCH; c++) {
+                if (b.nwork == b.wcap) return fail("sp_hipkv_decode_batch: more attention work items than the set's %s%lld", "", (long long)b.wcap);
+                hwork[b.nwork++] = make_int2(t, c);
+            }
         }
         // tokens, positions, page tables and work items lie in one block on both sides
         HIPCHK(hipMemcpyAsync(b.toks, htok, (size_t)((uint8_t *)(hwork + b.nwork) - (uint8_t *)htok), hipMemcpyHostToDevice,
