@@ -213,11 +213,12 @@ __device__ __forceinline__ float rne_u128_scaled(u128 mag, int k) {
 __device__ __forceinline__ float rne_i128_scaled(i128 v, int k) {
     return v >= 0 ? rne_u128_scaled((u128)v, k) : -rne_u128_scaled((u128)(-v), k);
 }
-// the conversion rounds to nearest even and the scaling is exact where the
-// result is a normal float; the general path takes the rest
+// The conversion rounds to nearest even and the scaling is exact above 2^-126; the
+// general path takes the rest.  (A sum scaled to 2^-126 itself may have been
+// rounded twice: 24 bits just below it are one more than a subnormal keeps.)
 __device__ __forceinline__ float rne_i64_scaled(int64_t v, int k) {
     const float f = ldexpf((float)v, k), m = fabsf(f);
-    if (m >= 0x1p-126f && m < INFINITY) return f;
+    if (m > 0x1p-126f && m < INFINITY) return f;
     return v >= 0 ? rne_u128_scaled((u128)(uint64_t)v, k) : -rne_u128_scaled((u128)(uint64_t)(-v), k);
 }
 // RNE of num / (den * 2^k), den > 0

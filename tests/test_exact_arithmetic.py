@@ -87,6 +87,15 @@ def test_scaled_rounding_is_nearest_even(dev):
     t = (np.int64(1) << rng.integers(24, 60, 3000)) + rng.integers(-3, 4, 3000) * (np.int64(1) << rng.integers(0, 36, 3000))
     v = np.concatenate([v, t, -t, [0]]).astype(np.int64)
     k = rng.integers(-200, 70, v.size).astype(np.int32)
+    # around 2^-126, where 24 bits of a value below it are one more than a float
+    # keeps: the midpoint to the largest subnormal (half), the one above it
+    # (quarter) and their neighbours, for several widths of the sum
+    for w in (26, 44, 61):
+        one = 1 << w
+        half, quarter = one >> 24, one >> 25
+        b = [one + o + d for o in (0, -quarter, -half, -half - quarter, -2 * half, quarter, half) for d in (-2, -1, 0, 1, 2)]
+        v = np.concatenate([v, b, -np.array(b)]).astype(np.int64)
+        k = np.concatenate([k, np.full(2 * len(b), -126 - w)]).astype(np.int32)
     o = np.empty(v.size, np.float32)
     dev.rne(p(v), p(k), v.size, p(o))
     for vi, ki, oi in zip(v.tolist(), k.tolist(), o.tolist()):
