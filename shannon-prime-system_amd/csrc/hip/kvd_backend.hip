@@ -11,6 +11,7 @@
 #include "sp_model_abi.h"
 #include "sp_hipkv.h"
 #include "kvd_internal.h"
+#include "kvd_batch.h"
 #include "kvd_spinor.h"
 #include <hip/hip_runtime.h>
 #include <algorithm>
@@ -21,6 +22,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -144,41 +146,6 @@ struct DevLayer {
     DevW q, k, v, o, gate, up, down;
     const float *attn_norm, *q_norm, *k_norm, *ffn_norm, *post_attn, *post_ffw;
 };
-// logits of a batched step leave through pinned slots (logits_to_host)
-constexpr int LOGIT_SLOTS = 4;
-constexpr size_t LOGIT_SLOT_BYTES = (size_t)1 << 20;
-
-// Buffers of the batched calls (prefill, batched decode): [tokens][...] rows, GEMM
-// operands, score grids.  A call leases one from its model and gives it back when
-// its stream has drained (BatchLease), so sessions that prefill one after the
-// other share one, and threads that run at once have one each.
-struct Batch {
-    int mode = 0, pmax = 0;              // its sizes serve this pmax and below; FLOAT's serve both modes
-    void *buf = nullptr;
-    int TB = 0, mcb = 0;                 // tokens per attention batch, chunk capacity per q-head
-    float *x0, *x1, *q, *k, *v, *qr, *ao, *ap, *hh, *dn, *rope, *part, *part_ml;
-    int8_t *planes; int *sh, *counter, *zs;
-    int64_t *vacc, *vacc_s;
-    int64_t *gpart; int *gcnt;           // GEMM split-K partial slices and tile arrival counters
-    // batched decode over sessions (allocated on first use): logits rows,
-    // greedy tokens, per-token token / position / per-layer page tables
-    void *dbuf = nullptr;
-    float *logits; int *next, *toks, *tpos; float *const **tpages;
-    int2 *work; int nwork = 0, wcap = 0;   // full-context layers' (token, chunk) work items
-    void *hstage = nullptr;              // pinned: toks/tpos/tpages/work as uploaded, then:
-    int *hnext = nullptr;                // the greedy tokens
-    uint8_t *hslots = nullptr;           // LOGIT_SLOTS pieces of logits on their way to the caller
-    hipEvent_t slot_ev[LOGIT_SLOTS] = {};
-    void release() {
-        if (buf) hipFree(buf);
-        if (dbuf) hipFree(dbuf);
-        if (hstage) hipHostFree(hstage);
-        for (hipEvent_t e : slot_ev) if (e) hipEventDestroy(e);
-        *this = Batch{};
-    }
-};
-constexpr size_t MAX_IDLE_BATCHES = 4;       // kept by a model; more go back to the device at once
-
 struct DevModel {
     const qwen3_model *qm = nullptr;
     int refs = 0, gemma = 0;
@@ -194,8 +161,7 @@ struct DevModel {
     // captured graphs intact): a fork or open with the same pmax and window ring
     // takes one instead of allocating; they hold no model reference
     std::vector<sp_kvdecode_handle *> shells;
-    std::mutex batch_mu;
-    std::vector<Batch> batches;               // idle, whole (every counter and total at zero)
+    BatchSets batches;
 };
 std::map<const qwen3_model *, DevModel *> g_models;
 void free_handle(sp_kvdecode_handle *h);
@@ -399,7 +365,7 @@ DevModel *model_get(const qwen3_model *qm, bool upload = true) {
     m->bytes = up.total;
     if (!upload) return m.release();
 
-    if (hipMalloc(&m->buf, up.total) != hipSuccess) {
+    if (dev_malloc(&m->buf, up.total) != hipSuccess) {
         fail("sp_hipkv_open: hipMalloc of %s%lld weight bytes failed", "", (long long)up.total); return nullptr;
     }
     uint8_t *base = (uint8_t *)m->buf;
@@ -436,7 +402,6 @@ void model_put(DevModel *m) {
     if (!m || --m->refs > 0) return;
     for (sp_kvdecode_handle *sh : m->shells) free_handle(sh);
     m->shells.clear();
-    for (Batch &b : m->batches) b.release();
     g_models.erase(m->qm);
     hipFree(m->buf);
     delete m;
@@ -496,7 +461,7 @@ struct KvPool {
     int grow(int min_pages) {
         const int n = std::max(min_pages, pages_per_chunk);
         void *c = nullptr;
-        if (hipMalloc(&c, (size_t)n * page_bytes) != hipSuccess) return 1;
+        if (dev_malloc(&c, (size_t)n * page_bytes) != hipSuccess) return 1;
         chunks.push_back(c);
         for (int i = 0; i < n; i++) {
             ptr.push_back((float *)((uint8_t *)c + (size_t)i * page_bytes));
@@ -648,7 +613,7 @@ int build_tables(sp_kvdecode_handle *h) {
     }
     if (h->d_pt) { hipFree(h->d_pt); h->d_pt = nullptr; }
     if (h->h_pt) { hipHostFree(h->h_pt); h->h_pt = nullptr; }
-    HIPCHK(hipMalloc(&h->d_pt, tot * sizeof(float *)), "page table alloc");
+    HIPCHK(dev_malloc(&h->d_pt, tot * sizeof(float *)), "page table alloc");
     HIPCHK(hipHostMalloc(&h->h_pt, tot * sizeof(float *), hipHostMallocDefault), "page table mirror alloc");
     for (size_t i = 0; i < tot; i++) h->h_pt[i] = nullptr;
     HIPCHK(hipMemcpyAsync(h->d_pt, h->h_pt, tot * sizeof(float *), hipMemcpyHostToDevice, h->stream), "page table init");
@@ -810,7 +775,7 @@ int alloc_scratch(sp_kvdecode_handle *h) {
     };
     size_t tot = 0;
     for (auto &it : items) tot = align_up(tot + it.n, 256);
-    HIPCHK(hipMalloc(&h->scratch, tot), "scratch alloc");
+    HIPCHK(dev_malloc(&h->scratch, tot), "scratch alloc");
     // cleared on the handle's stream: a null-stream memset is not ordered
     // before the handle's (non-blocking) kernels
     HIPCHK(hipMemsetAsync(h->scratch, 0, tot, h->stream), "scratch clear");
@@ -894,7 +859,7 @@ int alloc_recall(sp_kvdecode_handle *h, int B, int W, int sink, int r) {
     size_t tot = 0;
     for (auto &it : items) tot = align_up(tot + it.n, 256);
     void *buf = nullptr;
-    HIPCHK(hipMalloc(&buf, tot), "recall buffers alloc");
+    HIPCHK(dev_malloc(&buf, tot), "recall buffers alloc");
     R.buf = buf;
     size_t off = 0;
     for (auto &it : items) { *it.p = (uint8_t *)buf + off; off = align_up(off + it.n, 256); }
@@ -1154,29 +1119,12 @@ bool batch_supported(const sp_kvdecode_handle *h) {
 struct BatchLease {
     sp_kvdecode_handle *h;
     bool whole = false;
-    explicit BatchLease(sp_kvdecode_handle *hh) : h(hh) {
-        std::lock_guard<std::mutex> lk(h->m->batch_mu);
-        auto &v = h->m->batches;
-        for (size_t i = v.size(); i-- > 0;)
-            if ((v[i].mode == FLOAT || h->mode != FLOAT) && v[i].pmax >= h->pmax) { h->b = v[i]; v.erase(v.begin() + (ptrdiff_t)i); return; }
-        h->b.mode = h->mode; h->b.pmax = h->pmax;
-    }
+    explicit BatchLease(sp_kvdecode_handle *hh) : h(hh) { h->b = h->m->batches.take(h->mode == FLOAT, h->pmax); }
     BatchLease(const BatchLease &) = delete;
     void done() { whole = true; }             // after the stream's synchronize
     ~BatchLease() {
-        if (!whole) hipStreamSynchronize(h->stream);
-        Batch drop;
-        {
-            std::lock_guard<std::mutex> lk(h->m->batch_mu);
-            auto &v = h->m->batches;
-            drop = h->b;
-            if (whole && drop.buf) {
-                v.push_back(drop);
-                drop = Batch{};
-                if (v.size() > MAX_IDLE_BATCHES) { drop = v.front(); v.erase(v.begin()); }
-            }
-        }
-        drop.release();
+        if (!whole) { hipStreamSynchronize(h->stream); h->b.release(); }
+        else if (h->b.buf) h->m->batches.give(h->b);
         h->b = Batch{};
     }
 };
@@ -1200,13 +1148,14 @@ int alloc_batch(sp_kvdecode_handle *h) {
         {(void **)&b.sh, TG * 4}, {(void **)&b.counter, TB * m->NKV * 4},
         {(void **)&b.zs, TB * m->NH * (size_t)h->max_chunks * 16 * 4},
         {(void **)&b.part_ml, TB * m->NH * (size_t)b.mcb * 16},
-        {(void **)&b.part, h->mode == FLOAT ? TB * m->NH * (size_t)b.mcb * m->HD * 4 : 256},
+        {(void **)&b.part, b.flt ? TB * m->NH * (size_t)b.mcb * m->HD * 4 : 256},
         {(void **)&b.vacc, TB * QD * 8 * VREP}, {(void **)&b.vacc_s, TB * m->NH * 8 * VREP},
         {(void **)&b.gpart, GEMM_PART_BYTES}, {(void **)&b.gcnt, GEMM_TILE_COUNTERS * 4},
     };
     size_t tot = 0;
     for (auto &it : items) tot = align_up(tot + it.n, 256);
-    HIPCHK(hipMalloc(&b.buf, tot), "prefill batch alloc");
+    HIPCHK(dev_malloc(&b.buf, tot), "prefill batch alloc");
+    b.bytes = tot;
     HIPCHK(hipMemsetAsync(b.buf, 0, tot, h->stream), "prefill batch clear");     // ordered before the batch kernels
     size_t off = 0;
     for (auto &it : items) { *it.p = (uint8_t *)b.buf + off; off = align_up(off + it.n, 256); }
@@ -1554,9 +1503,9 @@ int sp_hipkv_prefill(sp_kvdecode_handle *h, const int32_t *tokens, int n_tok) {
     HIPCHK(hipStreamSynchronize(h->stream), "prefill staging");
     HIPCHK(hipMemcpyAsync(h->tokbuf + h->dpos, tokens, (size_t)n_tok * 4, hipMemcpyHostToDevice, h->stream),
            "prefill tokens");
-    std::unique_ptr<BatchLease> lease;
+    std::optional<BatchLease> lease;
     if (h->use_batch && batch_supported(h)) {
-        lease.reset(new BatchLease(h));
+        lease.emplace(h);
         if (alloc_batch(h)) return 1;
         // window layers on a ring: writing position q reuses the page slot of
         // the page ring_pages back, i.e. drops positions up to q - ring*PAGE + PAGE-1;
@@ -1656,7 +1605,7 @@ static int decode_batch_impl(sp_kvdecode_handle *const *hs, int n, const int32_t
         b.hnext = (int *)((uint8_t *)b.hstage + align_up(up, 4096));
         b.hslots = (uint8_t *)b.hnext + align_up(nb, 4096);
         for (hipEvent_t &e : b.slot_ev) if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming), "batch decode event");
-        HIPCHK(hipMalloc(&b.dbuf, align_up(lb, 256) + align_up(nb, 256) + up), "batch decode alloc");
+        HIPCHK(dev_malloc(&b.dbuf, align_up(lb, 256) + align_up(nb, 256) + up), "batch decode alloc");
         uint8_t *p = (uint8_t *)b.dbuf;
         b.logits = (float *)p; p += align_up(lb, 256);
         b.next = (int *)p; p += align_up(nb, 256);
