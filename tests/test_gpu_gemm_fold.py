@@ -18,7 +18,7 @@ def bits(a):
 # (share of the 32-column blocks scaled down, by 2^-k): none beyond the random
 # init's own; a listed share of deep low digits; more than the list takes; one
 # beyond the digits
-SPREADS = {"plain": (0.0, 0), "listed": (0.01, 7), "digit3": (0.2, 6), "per-block": (0.05, 12)}
+SPREADS = {"plain": (0.0, 0), "listed": (0.003, 7), "digit3": (0.2, 6), "per-block": (0.05, 12)}
 
 
 @pytest.mark.parametrize("spread", list(SPREADS))
