@@ -191,6 +191,13 @@ int  sp_hipkv_set_window_one_launch(sp_kvdecode_handle *h, int on);
  * GEMMs, token-batched attention) or one decode step per token (0).  Both
  * leave the same K/V (bit-identical in exact mode). */
 int  sp_hipkv_set_batch_prefill(sp_kvdecode_handle *h, int on);
+/* The shape of the batched passes' GEMM launches: workgroups of 8 / k_groups row
+ * groups x k_groups parts of K and token_tiles 16-token tiles ((1,1) (1,2) (1,4)
+ * (2,2) (2,4) (4,1) (4,2) (8,1)), K split over up to k_splits workgroups (1-16;
+ * fewer where K is too short).  0, 0, 0 (default): each launch's own choice, by
+ * estimated time.  Every shape gives the same bits; 4 token tiles are refused at
+ * the launch for weights that run three digits.  For tests and measurement. */
+int  sp_hipkv_set_gemm_shape(sp_kvdecode_handle *h, int k_groups, int token_tiles, int k_splits);
 /* Exact mode stores V as vq = rne(v * 2^16) clamped to +-(2^23 - 1), which
  * keeps the exact V-sum inside int64 (|v| below 128).  This counts the V heads
  * this handle stored with at least one clamped element since it was opened or

@@ -504,6 +504,7 @@ struct sp_kvdecode_handle {
     int mode = FLOAT, pmax = 0, dpos = 0, use_graph = 1, hwm = 0;
     int kvc = KVC_PLAIN;                     // KV codec (KVC_SPINOR: SP_KV_SPINOR sessions)
     int use_batch = 1;                       // batched (MFMA) prefill where the shapes allow it
+    GemmArgs::Shape gemm_shape{};            // of the folded GEMM (wk 0: the launch's plan)
     int max_rewind = 0;                      // 0: full tables for window layers
     int pool_growth = 0;                     // pages per pool growth (0: ~1 GiB)
     int recall_kvsel = 0;                    // SP_RECALL_KVSEL: one recall selection per kv head
@@ -1189,7 +1190,7 @@ int run_batch(sp_kvdecode_handle *h, int T, int pos0, int pos_hi, bool multi, Ti
     };
     auto gemm = [&](int cols, bool fold) {
         GemmArgs g{};
-        g.cols = cols; g.planes = b.planes; g.sh = b.sh; g.T = T; g.TP = tp(fold); g.fold = fold; g.mode = h->mode; g.act = ACT_NONE;
+        g.cols = cols; g.planes = b.planes; g.sh = b.sh; g.T = T; g.TP = tp(fold); g.fold = fold; g.mode = h->mode; g.act = ACT_NONE; g.shape = h->gemm_shape;
         g.part = b.gpart; g.part_cap = GEMM_PART_BYTES / 8; g.cnt = b.gcnt; g.cnt_cap = GEMM_TILE_COUNTERS;
         return g;
     };
@@ -1431,7 +1432,7 @@ int sp_hipkv_open(const void *qm_opaque, int pmax, sp_kvdecode_handle **out) {
         // a kept shell: reset to the open defaults, unmapped tables
         set_handle_mode(sh, FLOAT);
         if (sh->kvc != KVC_PLAIN) { sh->kvc = KVC_PLAIN; free_graphs(sh); }   // graphs bake in the codec
-        sh->use_graph = 1; sh->use_batch = 1; sh->dpos = 0; sh->hwm = 0; sh->pool_growth = 0;
+        sh->use_graph = 1; sh->use_batch = 1; sh->gemm_shape = {}; sh->dpos = 0; sh->hwm = 0; sh->pool_growth = 0;
         if (sh->recall_kvsel) { sh->recall_kvsel = 0; free_graphs(sh); }
         if (!sh->win_one) { sh->win_one = 1; free_graphs(sh); }
         sh->ring2 = 0;
@@ -1828,6 +1829,15 @@ int sp_hipkv_set_batch_prefill(sp_kvdecode_handle *h, int on) {
     return 0;
 }
 
+int sp_hipkv_set_gemm_shape(sp_kvdecode_handle *h, int k_groups, int token_tiles, int k_splits) {
+    if (!h) return fail("sp_hipkv_set_gemm_shape: null handle%s");
+    if (!k_groups && !token_tiles && !k_splits) { h->gemm_shape = {}; return 0; }
+    if (!gemm_fold_built(k_groups, token_tiles) || k_splits < 1 || k_splits > 16)
+        return fail("sp_hipkv_set_gemm_shape: no kernel of this shape%s");
+    h->gemm_shape = {k_groups, token_tiles, k_splits};
+    return 0;
+}
+
 int sp_hipkv_set_recall(sp_kvdecode_handle *h, int B, int W, int sink, int r) {
     if (!h) return fail("sp_hipkv_set_recall: null handle%s");
     if (B < 0 || W < 0 || sink < 0) return fail("sp_hipkv_set_recall: negative budget, window or sink count%s");
@@ -1928,7 +1938,7 @@ int sp_hipkv_fork(const sp_kvdecode_handle *p, sp_kvdecode_handle **out) {
     if (hipMemsetAsync(h->vclamp, 0, sizeof(int), h->stream) != hipSuccess) {
         sp_hipkv_close(h.release()); return fail("sp_hipkv_fork: clamp counter reset failed%s");
     }
-    h->use_batch = p->use_batch; h->use_graph = p->use_graph; h->pool_growth = p->pool_growth;
+    h->use_batch = p->use_batch; h->gemm_shape = p->gemm_shape; h->use_graph = p->use_graph; h->pool_growth = p->pool_growth;
     if (h->recall_kvsel != p->recall_kvsel) { h->recall_kvsel = p->recall_kvsel; free_graphs(h.get()); }
     if (h->win_one != p->win_one) { h->win_one = p->win_one; free_graphs(h.get()); }
     h->ring2 = p->ring2;

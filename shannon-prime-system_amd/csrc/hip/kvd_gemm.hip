@@ -475,6 +475,16 @@ static void fold_pick(const GemmArgs &g, int nd, int wk, int tt, dim3 grid, hipS
 // two slots, 10% more on a full chip; a workgroup 5 us around its steps, more
 // with the activation; a split 3 us and its share of the partial sums.
 static const int FOLD_SHAPES[][2] = {{1, 1}, {1, 2}, {1, 4}, {2, 2}, {2, 4}, {4, 1}, {4, 2}, {8, 1}};
+bool gemm_fold_built(int wk, int tt) {
+    for (const auto &sh : FOLD_SHAPES) if (sh[0] == wk && sh[1] == tt) return true;
+    return false;
+}
+// whether k splits of S super-steps each have some (of `slice` partial sums each)
+static bool split_ok(int k, int wk, int S, size_t slice, int wgs, size_t part_cap, int cnt_cap) {
+    if (k == 1) return true;
+    const int steps = (S + k * wk - 1) / (k * wk);
+    return k * wk <= S && slice * k <= part_cap && wgs <= cnt_cap && (S + steps * wk - 1) / (steps * wk) == k;
+}
 void fold_plan(int rows, int tiles, int S, bool paired, int nd, size_t slice, size_t part_cap, int cnt_cap, int &wk, int &tt, int &ks) {
     double best = 1e30;
     wk = 1; tt = 1; ks = 1;
@@ -485,9 +495,8 @@ void fold_plan(int rows, int tiles, int S, bool paired, int nd, size_t slice, si
         const int wgs = ((rows + rows_wg - 1) / rows_wg) * ((tiles + TT - 1) / TT);
         const double outs = (double)FOLD_WAVES / WK * 32 * 16 * TT;
         for (int k = 1; k <= 16; k++) {
-            if (k > 1 && (k * WK > S || slice * k > part_cap || wgs > cnt_cap)) break;
+            if (!split_ok(k, WK, S, slice, wgs, part_cap, cnt_cap)) continue;
             const int steps = (S + k * WK - 1) / (k * WK);
-            if (k > 1 && (S + steps * WK - 1) / (steps * WK) != k) continue;    // a split without super-steps
             const double full = wgs * k < 256 ? wgs * k / 256.0 : 1.0;
             const double step = (1.0 + 0.21 * nd * TT) * (fold_depth(WK, TT) > 2 ? 1.0 : 1.25) * (1.0 + 0.1 * full);
             const double fixed = 5.0 + (paired ? 1.0 + 2.0 * TT / WK : 0.0);
@@ -506,10 +515,21 @@ void launch_gemm_fold(const GemmArgs &a, int nrows_total, hipStream_t s) {
     int nd = 2, wk, tt, ks;
     for (int i = 0; i < a.nseg; i++) nd = std::max(nd, a.seg[i].w.fold);
     const bool can = a.part && a.cnt;
-    fold_plan(nrows_total, a.TP / 16, a.cols / 128, paired, nd, (size_t)a.TP * g.arows, can ? a.part_cap : 0, can ? a.cnt_cap : 0,
-              wk, tt, ks);
-    const int rows_wg = FOLD_WAVES / wk * (paired ? 16 : 32);
-    const dim3 grid((nrows_total + rows_wg - 1) / rows_wg, (a.TP / 16 + tt - 1) / tt, ks);
+    const int S = a.cols / 128, tiles = a.TP / 16;
+    const size_t slice = (size_t)a.TP * g.arows, part_cap = can ? a.part_cap : 0;
+    const int cnt_cap = can ? a.cnt_cap : 0;
+    auto grid_of = [&] {
+        const int rows_wg = FOLD_WAVES / wk * (paired ? 16 : 32);
+        return dim3((nrows_total + rows_wg - 1) / rows_wg, (tiles + tt - 1) / tt, ks);
+    };
+    if (a.shape.wk) {
+        wk = a.shape.wk; tt = a.shape.tt; ks = 1;
+        if (!gemm_fold_built(wk, tt) || (nd == 3 && tt == 4)) return launch_fail("folded GEMM: no kernel of the shape that was set");
+        const dim3 one = grid_of();
+        for (int k = 2; k <= a.shape.ks; k++)          // the most splits up to those set
+            if (split_ok(k, wk, S, slice, (int)(one.x * one.y), part_cap, cnt_cap)) ks = k;
+    } else fold_plan(nrows_total, tiles, S, paired, nd, slice, part_cap, cnt_cap, wk, tt, ks);
+    const dim3 grid = grid_of();
     if (paired) fold_pick<true>(g, nd, wk, tt, grid, s);
     else fold_pick<false>(g, nd, wk, tt, grid, s);
 }

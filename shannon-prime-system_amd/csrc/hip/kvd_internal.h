@@ -222,6 +222,9 @@ struct GemmArgs {
     size_t part_cap;   // int64 elements of part
     int cnt_cap;       // counters in cnt
     int arows;
+    // folded GEMM: the K groups, token tiles and K splits to run instead of the
+    // plan's (wk 0: the plan; sp_hipkv_set_gemm_shape)
+    struct Shape { int wk, tt, ks; } shape;
 };
 
 // Hand-off between workgroups of one launch without cache-wide fences: all data
@@ -288,6 +291,7 @@ int gemm_folds(const DevW &w);
 // (The random-init weights have 0.12% by themselves.)
 constexpr double FOLD_LIST_MAX = 0.0075;
 void launch_gemm_fold(const GemmArgs &a, int nrows_total, hipStream_t s);
+bool gemm_fold_built(int wk, int tt);
 void launch_advance(DState *st, hipStream_t s);
 void launch_gemv(const GemvArgs &a, int nrows_total, hipStream_t s);
 void gemv_time_next(hipEvent_t start, hipEvent_t stop);   // events of the calling thread's next GEMV launch

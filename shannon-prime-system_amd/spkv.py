@@ -121,6 +121,7 @@ def kv():
         _sig(lib, "sp_hipkv_ring2_stats", c_int, [c_void_p, c_void_p])
         _sig(lib, "sp_hipkv_write_kv", c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p])
         _sig(lib, "sp_hipkv_set_batch_prefill", c_int, [c_void_p, c_int])
+        _sig(lib, "sp_hipkv_set_gemm_shape", c_int, [c_void_p, c_int, c_int, c_int])
         _sig(lib, "sp_hipkv_fork", c_int, [c_void_p, ctypes.POINTER(c_void_p)])
         _sig(lib, "sp_hipkv_attach", c_int, [c_void_p, c_int, c_int])
         _sig(lib, "sp_hipkv_greedy", c_int, [c_void_p, c_int32, c_int, c_void_p, ctypes.POINTER(c_double)])

@@ -18,6 +18,9 @@ SMALL = {
                          head_dim=256, n_ff=1024, vocab=2048, swa_window=32),
     "qwen3-g4": dict(arch_id=spkv.ARCH_QWEN3, n_layers=2, hidden=512, n_heads=8, n_kv_heads=2,
                      head_dim=128, n_ff=1024, vocab=2048, untied=1),
+    # 384 q/k/v rows and 2112 vocabulary rows: not whole 256-row GEMM tiles
+    "qwen3-ragged": dict(arch_id=spkv.ARCH_QWEN3, n_layers=2, hidden=768, n_heads=4, n_kv_heads=1,
+                         head_dim=64, n_ff=1280, vocab=2112),
     # wide rows: the GEMVs split their columns over workgroups (2-3 splits, the
     # last one ragged) and combine exact partials atomically
     "qwen3-wide": dict(arch_id=spkv.ARCH_QWEN3, n_layers=2, hidden=2304, n_heads=8, n_kv_heads=4,
@@ -138,26 +141,61 @@ def oracle_ppl(o, toks, n_warm):
     return math.exp(nll / ns)
 
 
-def write_scaled(dirpath, name, share, down):
-    """The SMALL model `name` with a seeded `share` of every matrix's 32-column
-    block scales multiplied by 2^-down in the file (exact in f16 down to its
-    smallest step): returns the paths and the shape."""
+def _bscales(spm):
+    """A writable map of a model file, and the offset and size of every matrix's block scales."""
+    raw = np.memmap(spm, dtype=np.uint8, mode="r+")
+    count = int(raw[316:320].view(np.uint32)[0])
+    table, data = (int(x) for x in raw[320:336].view(np.uint64))
+    at = {}
+    for i in range(count):
+        e = raw[table + 256 * i:table + 256 * (i + 1)]
+        name = bytes(e[:80]).split(b"\0")[0].decode()
+        if name.endswith(".weight.bscale"):
+            off, size = (int(x) for x in e[152:168].copy().view(np.uint64))
+            at[name[:-len(".weight.bscale")]] = (data + off, size)
+    return raw, at
+
+
+def write_scaled(dirpath, name, share, down, only=None, max_context=512):
+    """The SMALL model `name` with a seeded `share` of the 32-column block scales
+    of every matrix (`only`: of those whose names hold one of these) multiplied by
+    2^-down in the file (exact in f16 down to its smallest step): returns the
+    paths and the shape."""
     d = SMALL[name]
-    prefix = os.path.join(str(dirpath), f"{name}_x{share}_{down}")
+    prefix = os.path.join(str(dirpath), f"{name}_x{share}_{down}_{'-'.join(only or ())}_c{max_context}")
     spm, spt = prefix + ".spm", prefix + ".spt"
     if not os.path.exists(spm):
-        spkv.write_model(prefix, max_context=512, **d)
-        raw = np.memmap(spm, dtype=np.uint8, mode="r+")
-        count = int(raw[316:320].view(np.uint32)[0])
-        table, data = (int(x) for x in raw[320:336].view(np.uint64))
+        spkv.write_model(prefix, max_context=max_context, **d)
+        raw, at = _bscales(spm)
         rng = np.random.default_rng(5)
-        for i in range(count):
-            e = raw[table + 256 * i:table + 256 * (i + 1)]
-            if bytes(e[:80]).split(b"\0")[0].endswith(b".bscale") and share:
-                off, size = (int(x) for x in e[152:168].copy().view(np.uint64))
-                sc = raw[data + off:data + off + size].view(np.float16)
+        for tensor, (off, size) in at.items():
+            if share and (only is None or any(o in tensor for o in only)):
+                sc = raw[off:off + size].view(np.float16)
                 pick = rng.random(sc.size) < share
                 sc[pick] = (sc[pick].astype(np.float32) * np.float32(2.0 ** -down)).astype(np.float16)
         raw.flush()
         del raw
     return spm, spt, d
+
+
+def gemm_forms(spm, d):
+    """The batched GEMM's form for each matrix of a model file: 0 per-block (a row's
+    non-zero scales span more than 9 exponents), 2 two digits and a list of the
+    blocks whose scale f16 2^(9 - row's largest exponent) has a low byte (at most
+    0.75% of them), 3 three digits."""
+    raw, at = _bscales(spm)
+    cols = {"attn_output": d["n_heads"] * d["head_dim"], "ffn_down": d["n_ff"]}
+    forms = {}
+    for tensor, (off, size) in at.items():
+        b = raw[off:off + size].view(np.uint16).reshape(-1, cols.get(tensor.split(".")[-1], d["hidden"]) // 32).astype(np.int64)
+        exp, mant = (b >> 10) & 31, b & 1023
+        sig = np.where(exp > 0, 1024 + mant, mant)
+        e = np.where(exp > 0, exp - 25, -24)
+        hi = np.where(sig > 0, e, -99).max(1, keepdims=True)
+        assert (b >> 15).max() == 0
+        if (np.where(sig > 0, hi - e, 0) > 9).any():
+            forms[tensor] = 0
+        else:
+            low = ((sig << np.maximum(e + 9 - hi, 0)) & 255) > 0
+            forms[tensor] = 2 if low.mean() <= 0.0075 else 3
+    return forms
