@@ -1233,7 +1233,9 @@ int run_batch(sp_kvdecode_handle *h, int T, int pos0, int pos_hi, bool multi, Ti
         // chunks of the batch's longest span: a window of W positions covers at
         // most (W-1)/chunk + 2 chunks whatever its alignment
         TM(a.win >= 0 ? 6 : 5, true);
-        if (!multi) a.part_tokens = b.TB;
+        // by the handle's own pmax, not the leased set's (no smaller): a call's
+        // sums must not depend on what other sessions left
+        if (!multi) a.part_slots = b.TB * (h->pmax / 64 + 2);
         if (prefill_attention_float(a)) launch_prefill_float(a, s);
         else for (int t = 0; t < T; t += b.TB) {                // one pass for a batched decode
             AttnArgs c = a;

@@ -111,7 +111,7 @@ struct AttnArgs {
     // batched prefill: nt tokens at positions pos0.. (token = blockIdx.y of
     // qk_prep, blockIdx.z of attention); every per-token buffer is [nt][...]
     int nt, pos0, rope_stride;
-    int part_tokens;         // float prefill: tokens the part / part_ml buffers hold at max_chunks each (0: the per-token kernels)
+    int part_slots;          // float prefill: parts of a q head, over all tokens, to split into at most (0: the per-token kernels)
     // batched decode over several sessions: token t's position and this
     // layer's page table (NULL: pos0 + t and `pages`)
     const int *tpos;

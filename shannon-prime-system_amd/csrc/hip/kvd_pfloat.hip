@@ -259,9 +259,11 @@ static void pfloat_go(const AttnArgs &a, hipStream_t s) {
     constexpr int TOK = PF_ROWS / G;
     const int tiles = (a.nt + TOK - 1) / TOK;
     // splits: two workgroups' worth of positions per CU, at least two tiles
-    // each, as many as the parts' buffers hold
+    // each, as many as the parts' buffers hold.  They are cut by this launch's
+    // tokens, so another cut of the same prompt adds its float sums in another
+    // order (about 1e-6 of the result).
     const int span = (a.pos0 + a.nt - 1) / PF_POS - start_of(a, a.nt > TOK ? a.nt - TOK : 0) / PF_POS + 1;
-    const int room = (int)std::min<size_t>((size_t)a.part_tokens * a.max_chunks / a.nt, 64);
+    const int room = std::min(a.part_slots / a.nt, 64);
     int n = (512 + tiles * a.NKV - 1) / (tiles * a.NKV);
     n = std::max(1, std::min(std::min(n, span / 2), room));
     const dim3 grid(a.NKV, tiles, n), wg(64 * PF_WAVES);
@@ -271,7 +273,7 @@ static void pfloat_go(const AttnArgs &a, hipStream_t s) {
 
 bool prefill_attention_float(const AttnArgs &a) {
     const int G = a.NH / a.NKV;
-    return a.mode == FLOAT && a.kvc == KVC_PLAIN && a.nt > 0 && !a.tpages && !a.tpos && a.part_tokens > 0 &&
+    return a.mode == FLOAT && a.kvc == KVC_PLAIN && a.nt > 0 && !a.tpages && !a.tpos && a.part_slots > 0 &&
            (a.HD == 64 || a.HD == 128 || a.HD == 256) && (G == 2 || G == 4);
 }
 

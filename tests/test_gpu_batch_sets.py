@@ -43,3 +43,26 @@ def test_a_short_batch_leaves_room_for_long_sessions(tmpdir_models):
     for b in bs + short + [long]:
         b.close()
     s.close(); m.close()
+
+
+def test_float_prefill_does_not_depend_on_the_set(tmpdir_models):
+    """A float prefill's position splits come from its own handle: the same bits
+    on a set of its own and on the larger one another session left."""
+    name, n = "gemma3-tiny", 600
+    spm, spt = model_files(tmpdir_models, name, max_context=4160)
+    V, NL = SMALL[name]["vocab"], SMALL[name]["n_layers"]
+    kvd = SMALL[name]["n_kv_heads"] * SMALL[name]["head_dim"]
+    out = []
+    for larger in (False, True):
+        m = spkv.Model(spm, spt)
+        s = spkv.Session(m, 64)
+        qm = spkv.l1().sp_session_qwen3_model(s.h)
+        big = spkv.Backend(qm, 4160)
+        if larger:
+            big.prefill(prompt(70, V, seed=1))
+        b = spkv.Backend(qm, 640)
+        b.prefill(prompt(n, V, seed=2))
+        out.append([b.read_kv(l, 0, n, kvd) for l in range(NL)])
+        b.close(); big.close(); s.close(); m.close()
+    for l, ((k0, v0), (k1, v1)) in enumerate(zip(*out)):
+        assert np.array_equal(k0.view(np.uint32), k1.view(np.uint32)) and np.array_equal(v0.view(np.uint32), v1.view(np.uint32)), l
