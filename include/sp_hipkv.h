@@ -189,7 +189,10 @@ int  sp_hipkv_set_graph(sp_kvdecode_handle *h, int on);
 int  sp_hipkv_set_window_one_launch(sp_kvdecode_handle *h, int on);
 /* Prefill through the batched path (1, default: 512 tokens per pass, int8-MFMA
  * GEMMs, token-batched attention) or one decode step per token (0).  Both
- * leave the same K/V (bit-identical in exact mode). */
+ * leave the same K/V: bit-identical in exact mode; in float mode to the order of
+ * the f32 sums.  That order depends on the tokens of the call and on the handle's
+ * pmax (positions are split over workgroups), so one prompt prefilled in other
+ * pieces, or step by step, agrees to about 2e-6 and not bit for bit. */
 int  sp_hipkv_set_batch_prefill(sp_kvdecode_handle *h, int on);
 /* The shape of the batched passes' GEMM launches: workgroups of 8 / k_groups row
  * groups x k_groups parts of K and token_tiles 16-token tiles ((1,1) (1,2) (1,4)

@@ -261,7 +261,7 @@ static void pfloat_go(const AttnArgs &a, hipStream_t s) {
     // splits: two workgroups' worth of positions per CU, at least two tiles
     // each, as many as the parts' buffers hold.  They are cut by this launch's
     // tokens, so another cut of the same prompt adds its float sums in another
-    // order (about 1e-6 of the result).
+    // order (up to 2e-6 of K, V and logits).
     const int span = (a.pos0 + a.nt - 1) / PF_POS - start_of(a, a.nt > TOK ? a.nt - TOK : 0) / PF_POS + 1;
     const int room = std::min(a.part_slots / a.nt, 64);
     int n = (512 + tiles * a.NKV - 1) / (tiles * a.NKV);
