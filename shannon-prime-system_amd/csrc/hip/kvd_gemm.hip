@@ -23,36 +23,15 @@
 #include "kvd_internal.h"
 #include "kvd_exact.h"
 #include "kvd_vec.h"
+#include "kvd_pass.h"
 #include <algorithm>
 
 namespace kvd {
 
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef short s2 __attribute__((ext_vector_type(2)));
 
-// raw buffer descriptor of [base, base + bytes): reads past it return zero
-__device__ __forceinline__ v4i rsrc_of(const void *base, uint32_t bytes) {
-    const uint64_t b = (uint64_t)base;
-    v4i r;
-    r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-    r.y = __builtin_amdgcn_readfirstlane((int)((uint32_t)(b >> 32) & 0xFFFFu));
-    r.z = __builtin_amdgcn_readfirstlane((int)bytes);
-    r.w = 0x00020000;                                  // 32-bit data format, stride 0
-    return r;
-}
-// Loads straight into LDS (no registers): lane l's bytes at voff + soff go to
-// LDS byte lds + 16 l (dma16) or, zero-extended, lds + 4 l (dma2).  The caller
-// counts them (vmcnt) and waits before anyone reads the bytes.
-__device__ __forceinline__ void dma16(uint32_t lds, int voff, v4i rsrc, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-__device__ __forceinline__ void dma2(uint32_t lds, int voff, v4i rsrc, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_ushort %1, %2, %3 offen lds"
-                 : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
 // all but this wave's youngest N loads have arrived and its LDS reads are done,
 // then the workgroup's barrier
 template <int N> __device__ __forceinline__ void arrive_barrier() {

@@ -38,29 +38,18 @@
 #include "kvd_exact.h"
 #include "kvd_vec.h"
 #include "kvd_spinor.h"
+#include "kvd_pass.h"
 #include <type_traits>
 
 namespace kvd {
 
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-
 constexpr int PS_CH = 64;            // positions per score workgroup (and per chunk maximum)
 constexpr int PV_CH = 2048;          // positions per V-sum workgroup (full-context layers)
 constexpr int PV_SUB = 512;          // ... in sub-chunks of 128 rows per wave (FP64 sums below 2^53)
 constexpr int DIG_MAX = 127 * (1 + 256 + 65536 + 16777216);   // largest |x| of four balanced digits
 constexpr int DIG3_MAX = 127 * (1 + 256 + 65536);             // ... of three
-
-__device__ __forceinline__ const float *pg(const AttnArgs &a, int pos) {
-    const int lp = pos / PAGE;
-    return gmem(a.pages)[a.ring_pages ? lp % a.ring_pages : lp];
-}
-// the first position token t of the batch attends
-__host__ __device__ __forceinline__ int win_start(const AttnArgs &a, int t) {
-    const int q = a.pos0 + t - a.win + 1;
-    return a.win >= 0 && q > 0 ? q : 0;
-}
 
 // x = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3, d in [-128, 127] (|x| <= DIG_MAX), the
 // digits as bytes: adding 128 to each byte place with carries gives d + 128
@@ -131,7 +120,7 @@ __global__ __launch_bounds__(256) void k_pattn_scores(AttnArgs a) {
     // and a copy of a row changes no range check)
     static_assert(PS_CH == PAGE && PS_CH * (HD / 16) % 256 == 0, "one page per chunk, whole row pieces per thread");
     constexpr int KIT = PS_CH * (HD / 16) / 256;
-    const int32_t *kpage = (const int32_t *)pg(a, cs) + (size_t)h * PAGE * HD;
+    const int32_t *kpage = (const int32_t *)page_at(a, cs) + (size_t)h * PAGE * HD;
     int4 kx[KIT][4];
     #pragma unroll
     for (int it = 0; it < KIT; it++) {
@@ -211,7 +200,7 @@ __global__ __launch_bounds__(256) void k_pattn_scores(AttnArgs a) {
                 const int tt = t0 + wave * TPW + mm / G;
                 if (tt >= a.nt || p > pos_hi) continue;
                 const float *q2 = a.qr + (size_t)tt * QD + (size_t)(h * G + mm % G) * HD;
-                const int32_t *krow = (const int32_t *)pg(a, p) + ((size_t)h * PAGE + (p & (PAGE - 1))) * HD;
+                const int32_t *krow = (const int32_t *)page_at(a, p) + ((size_t)h * PAGE + (p & (PAGE - 1))) * HD;
                 int64_t s = 0;
                 for (int d = 0; d < HD; d++) s += (int64_t)(int32_t)rintf(q2[d] * 65536.0f) * gmem(krow)[d];
                 ip[i] = s;
@@ -344,7 +333,7 @@ __global__ __launch_bounds__(WIN ? 512 : 256) void k_pattn_vsum(AttnArgs a) {
         auto load_v = [&](int j0, int32_t (&v)[UV][EPL]) {
             const int pa = __builtin_amdgcn_readfirstlane(cs + sb + (j0 < ns ? j0 : ns - 1));
             const int pb = __builtin_amdgcn_readfirstlane(cs + sb + (j0 + UV - 1 < ns ? j0 + UV - 1 : ns - 1));
-            const int32_t *ba = (const int32_t *)pg(a, pa) + voff, *bb = (const int32_t *)pg(a, pb) + voff;
+            const int32_t *ba = (const int32_t *)page_at(a, pa) + voff, *bb = (const int32_t *)page_at(a, pb) + voff;
             #pragma unroll
             for (int u = 0; u < UV; u++) {
                 const int p = __builtin_amdgcn_readfirstlane(cs + sb + (j0 + u < ns ? j0 + u : ns - 1));

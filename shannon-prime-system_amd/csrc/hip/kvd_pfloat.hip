@@ -21,40 +21,18 @@
 #include "kvd_internal.h"
 #include "kvd_vec.h"
 #include "kvd_spinor.h"
+#include "kvd_pass.h"
 #include <algorithm>
 
 namespace kvd {
 
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int PF_WAVES = 8, PF_ROWS = 16 * PF_WAVES;   // token-heads per workgroup
 constexpr int PF_POS = 32;                             // positions per tile (within one page)
 
-__device__ __forceinline__ const uint8_t *page_at(const AttnArgs &a, int pos) {
-    const int lp = pos / PAGE;
-    return (const uint8_t *)gmem(a.pages)[a.ring_pages ? lp % a.ring_pages : lp];
-}
-__host__ __device__ __forceinline__ int start_of(const AttnArgs &a, int t) {   // the first position token t attends
-    const int q = a.pos0 + t - a.win + 1;
-    return a.win >= 0 && q > 0 ? q : 0;
-}
-// raw buffer descriptor of [base, base + bytes)
-__device__ __forceinline__ v4i rsrc_of(const void *base, uint32_t bytes) {
-    const uint64_t b = (uint64_t)base;
-    v4i r;
-    r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-    r.y = __builtin_amdgcn_readfirstlane((int)((uint32_t)(b >> 32) & 0xFFFFu));
-    r.z = __builtin_amdgcn_readfirstlane((int)bytes);
-    r.w = 0x00020000;                                  // 32-bit data format, stride 0
-    return r;
-}
-// lane l's 16 bytes at voff go to LDS byte lds + 16 l (counted by vmcnt)
-__device__ __forceinline__ void dma16(uint32_t lds, int voff, v4i rsrc) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(lds), "v"(voff), "s"(rsrc) : "memory");
-}
 __device__ __forceinline__ bool finite4(const v4f &v) {
     const v4i b = __builtin_bit_cast(v4i, v) & 0x7F800000;
     return b.x != 0x7F800000 && b.y != 0x7F800000 && b.z != 0x7F800000 && b.w != 0x7F800000;
@@ -73,15 +51,15 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void k_pfloat(AttnArgs a, int nsp
     const int l16 = lane & 15, g = lane >> 4, h = blockIdx.x;
     const int t0 = (int)blockIdx.y * TOK, tend = t0 + TOK < a.nt ? t0 + TOK : a.nt;
     // this split's tiles of the token tile's span [start, last]
-    const int last = a.pos0 + tend - 1, lo = start_of(a, t0) / PF_POS, hi = last / PF_POS + 1;
+    const int last = a.pos0 + tend - 1, lo = win_start(a, t0) / PF_POS, hi = last / PF_POS + 1;
     const int per = (hi - lo + nsplit - 1) / nsplit, b0 = lo + (int)blockIdx.z * per, b1 = b0 + per < hi ? b0 + per : hi;
     // this lane's token-head, and the wave's token range
     const int row = wave * 16 + l16, tq = t0 + row / G, head = h * G + row % G;
     const bool live = tq < tend;
     const int wt0 = t0 + wave * 16 / G, wt1 = t0 + (wave * 16 + 15) / G < tend ? t0 + (wave * 16 + 15) / G : tend - 1;
-    const int my_lo = start_of(a, tq), my_hi = live ? a.pos0 + tq : -1;     // positions this token-head attends
-    const int w_lo = start_of(a, wt0), w_hi = a.pos0 + wt1;                 // ... any of the wave's
-    const int w_lo1 = start_of(a, wt1), w_hi0 = a.pos0 + wt0;               // ... all of them
+    const int my_lo = win_start(a, tq), my_hi = live ? a.pos0 + tq : -1;     // positions this token-head attends
+    const int w_lo = win_start(a, wt0), w_hi = a.pos0 + wt1;                 // ... any of the wave's
+    const int w_lo1 = win_start(a, wt1), w_hi0 = a.pos0 + wt0;               // ... all of them
     const bool wlive = wt0 < tend;
     const size_t QD = (size_t)a.NH * HD;
     v4f Q[CPR];                                                        // dims 16 s + 4 g ..
@@ -95,7 +73,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void k_pfloat(AttnArgs a, int nsp
     // (p % 16); rows past the batch's last position repeat it
     auto load = [&](int tile, int buf) {
         constexpr int N = PIECES / 64 / PF_WAVES;      // 1 KiB loads per wave of K, and of V
-        const uint8_t *page = page_at(a, __builtin_amdgcn_readfirstlane(tile * PF_POS));
+        const uint8_t *page = (const uint8_t *)page_at(a, __builtin_amdgcn_readfirstlane(tile * PF_POS));
         const int lp = last - tile * PF_POS, q0 = (tile * PF_POS) & (PAGE - 1);
         #pragma unroll
         for (int v = 0; v < 2; v++) {
@@ -262,7 +240,7 @@ static void pfloat_go(const AttnArgs &a, hipStream_t s) {
     // each, as many as the parts' buffers hold.  They are cut by this launch's
     // tokens, so another cut of the same prompt adds its float sums in another
     // order (up to 2e-6 of K, V and logits).
-    const int span = (a.pos0 + a.nt - 1) / PF_POS - start_of(a, a.nt > TOK ? a.nt - TOK : 0) / PF_POS + 1;
+    const int span = (a.pos0 + a.nt - 1) / PF_POS - win_start(a, a.nt > TOK ? a.nt - TOK : 0) / PF_POS + 1;
     const int room = std::min(a.part_slots / a.nt, 64);
     int n = (512 + tiles * a.NKV - 1) / (tiles * a.NKV);
     n = std::max(1, std::min(std::min(n, span / 2), room));
