@@ -1,6 +1,8 @@
 """The buffers that batched calls of one model lease from each other: a call
 with short contexts may take the set of one with long contexts, and what it adds
 to that set serves the long ones afterwards."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -66,3 +68,54 @@ def test_float_prefill_does_not_depend_on_the_set(tmpdir_models):
         b.close(); big.close(); s.close(); m.close()
     for l, ((k0, v0), (k1, v1)) in enumerate(zip(*out)):
         assert np.array_equal(k0.view(np.uint32), k1.view(np.uint32)) and np.array_equal(v0.view(np.uint32), v1.view(np.uint32)), l
+
+
+def test_calls_of_several_threads_modes_and_lengths(tmpdir_models):
+    """Prefills and batched steps of handles with their own pmax and mode, from
+    four threads at once on one model's sets, leave the bits of the same calls
+    one after another."""
+    name = "gemma3-w200"
+    spm, spt = model_files(tmpdir_models, name, max_context=2048)
+    V, NL = SMALL[name]["vocab"], SMALL[name]["n_layers"]
+    kvd = SMALL[name]["n_kv_heads"] * SMALL[name]["head_dim"]
+    m = spkv.Model(spm, spt)
+    s = spkv.Session(m, 64)
+    qm = spkv.l1().sp_session_qwen3_model(s.h)
+    jobs = [(1600, True, 700), (300, False, 280), (640, False, 600), (64, True, 50)]
+
+    def work(i, reps):
+        pmax, exact, n = jobs[i]
+        bs = [spkv.Backend(qm, pmax, exact=exact) for _ in range(2)]
+        pr, toks = prompt(n, V, seed=40 + i), prompt(2, V, seed=50 + i)
+        out = []
+        for _ in range(reps):
+            for b in bs:
+                b.prefill(pr)
+            lg, nxt = spkv.Backend.decode_batch(bs, toks, V)
+            out.append([lg, nxt] + [x for l in range(NL) for x in bs[1].read_kv(l, 0, n, kvd)])
+            for b in bs:
+                b.rewind(n + 1)
+        for b in bs:
+            b.close()
+        return out
+
+    want = [work(i, 1)[0] for i in range(len(jobs))]
+    got, errs = [None] * len(jobs), []
+
+    def run(i):
+        try:
+            got[i] = work(i, 4)
+        except Exception as e:                          # shown below
+            errs.append((i, e))
+
+    th = [threading.Thread(target=run, args=(i,)) for i in range(len(jobs))]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not errs, errs
+    for i, reps in enumerate(got):
+        for r, o in enumerate(reps):
+            for j, (x, y) in enumerate(zip(o, want[i])):
+                assert np.array_equal(x.view(np.uint32), y.view(np.uint32)), (i, r, j)
+    s.close(); m.close()
